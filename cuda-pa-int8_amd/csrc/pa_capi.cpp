@@ -664,7 +664,7 @@ pa_status_t quant_write(const void* key, const void* value, int64_t key_token_st
       x, 16);
   if (st != PA_OK || num_tokens == 0) return st;
   if (!k_scales || !v_scales) return PA_ERR_NULL_POINTER;
-  pa::QuantLaunch l{};
+  pa::WriteLaunch l{};
   l.key = key;
   l.value = value;
   l.key_token_stride = key_token_stride;
@@ -683,9 +683,13 @@ pa_status_t quant_write(const void* key, const void* value, int64_t key_token_st
   l.v_scale_in = v_scale_in;
   l.num_blocks = num_blocks;
   l.block_size = block_size;
-  l.bf16_input = bf16_input;
   l.stream = reinterpret_cast<hipStream_t>(stream);
-  return pa::launch_quant_write_i8(l) == hipSuccess ? PA_OK : PA_ERR_LAUNCH;
+  const bool given = k_scale_in != nullptr;
+  const hipError_t e = given ? (bf16_input ? pa::launch_quant_write_i8<1, 1>(l)
+                                           : pa::launch_quant_write_i8<1, 0>(l))
+                             : (bf16_input ? pa::launch_quant_write_i8<0, 1>(l)
+                                           : pa::launch_quant_write_i8<0, 0>(l));
+  return e == hipSuccess ? PA_OK : PA_ERR_LAUNCH;
 }
 
 }  // namespace
@@ -758,7 +762,7 @@ pa_status_t pa_reshape_and_cache_f16(const void* key, const void* value,
       slot_mapping, num_tokens, num_kv_heads, head_dim, k_cache, v_cache, num_blocks, block_size,
       x, 8);
   if (st != PA_OK || num_tokens == 0) return st;
-  pa::CacheWriteLaunch l{};
+  pa::WriteLaunch l{};
   l.key = key;
   l.value = value;
   l.key_token_stride = key_token_stride;

@@ -151,7 +151,9 @@ PA_FOR_EACH_HEAD_DIM(PA_DECLARE_DECODE_D)
 // (pa_fill.hip).  A HIP graph may capture it: no memset node is recorded.
 hipError_t launch_fill_zero(void* p, size_t bytes, hipStream_t stream);
 
-struct QuantLaunch {
+// One paged-cache write: fp16 placement, or INT8 with per-token scales or
+// one given scale per tensor.
+struct WriteLaunch {
   const void* key;
   const void* value;
   int64_t key_token_stride;
@@ -164,7 +166,7 @@ struct QuantLaunch {
   int head_dim;
   void* k_cache;
   void* v_cache;
-  float* k_scales;
+  float* k_scales;   // INT8 (NULL for the fp16 write)
   float* v_scales;
   // Per-tensor mode: one given fp32 scale for every K (V) element, read on
   // the device; both NULL for the per-token mode.
@@ -172,32 +174,18 @@ struct QuantLaunch {
   const float* v_scale_in;
   int num_blocks;
   int block_size;
-  bool bf16_input;   // key / value are bf16 (else fp16)
   hipStream_t stream;
 };
 
-// Defined in pa_quant.hip.
-hipError_t launch_quant_write_i8(const QuantLaunch& l);
-
-struct CacheWriteLaunch {
-  const void* key;
-  const void* value;
-  int64_t key_token_stride;
-  int64_t key_head_stride;
-  int64_t value_token_stride;
-  int64_t value_head_stride;
-  const int64_t* slot_mapping;
-  int num_tokens;
-  int num_kv_heads;
-  int head_dim;
-  void* k_cache;
-  void* v_cache;
-  int num_blocks;
-  int block_size;
-  hipStream_t stream;
-};
-
-// Defined in pa_cache_write.hip.
-hipError_t launch_cache_write_f16(const CacheWriteLaunch& l);
+// INT8 write with per-token scales or one given scale per tensor, from fp16 or
+// bf16 rows (one specialization per compilation of pa_quant.hip), and the fp16
+// write (pa_cache_write.hip).
+template <int GIVEN_SCALE, int BF16>
+hipError_t launch_quant_write_i8(const WriteLaunch& l);
+template <> hipError_t launch_quant_write_i8<0, 0>(const WriteLaunch& l);
+template <> hipError_t launch_quant_write_i8<0, 1>(const WriteLaunch& l);
+template <> hipError_t launch_quant_write_i8<1, 0>(const WriteLaunch& l);
+template <> hipError_t launch_quant_write_i8<1, 1>(const WriteLaunch& l);
+hipError_t launch_cache_write_f16(const WriteLaunch& l);
 
 }  // namespace pa

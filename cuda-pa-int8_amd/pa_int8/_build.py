@@ -38,11 +38,12 @@ PROBE_LIB_NAME = "libpa_bench_probe.so"
 # entry (keep in step with PA_FOR_EACH_HEAD_DIM in csrc/pa_internal.hpp).
 HEAD_DIMS = tuple(range(8, 257, 8))
 HIP_SOURCES = [
-    "pa_quant.hip",
     "pa_cache_write.hip",
     "pa_fill.hip",
     "pa_noalloc.hip",
 ]
+# pa_quant.hip is compiled once per (scale mode, input type).
+QUANT_VARIANTS = tuple((given, bf16) for given in (0, 1) for bf16 in (0, 1))
 HOST_SOURCES = ["pa_capi.cpp"]
 PROBE_SOURCES = ["bench/pa_probe.hip", "bench/pa_probe_decode.hip", "bench/pa_probe_write.hip"]
 
@@ -104,6 +105,11 @@ def build_library(verbose=False, jobs=None):
         obj = os.path.join(OBJ_DIR, f"pa_decode_d{d}.o")
         objs.append(obj)
         cmds.append(_compile_cmd("pa_decode_inst.hip", obj, [f"-DPA_HEAD_DIM={d}"]))
+    for given, bf16 in QUANT_VARIANTS:
+        obj = os.path.join(OBJ_DIR, f"pa_quant_{given}{bf16}.o")
+        objs.append(obj)
+        cmds.append(_compile_cmd("pa_quant.hip", obj,
+                                 [f"-DPA_QUANT_GIVEN={given}", f"-DPA_QUANT_BF16={bf16}"]))
     for src in HIP_SOURCES + HOST_SOURCES:
         obj = os.path.join(OBJ_DIR, os.path.splitext(src)[0] + ".o")
         objs.append(obj)

@@ -1,6 +1,6 @@
 """CPU check of the arithmetic the quantize kernel uses (no GPU needed).
 
-The kernel (cuda-pa-int8_amd/csrc/pa_quant.hip) computes the per-token scale
+The kernel (cuda-pa-int8_amd/csrc/pa_write_kernel.hpp) computes the per-token scale
 as fp16(fl(a * fl(1/127))) and q = rne(x / s) through y = x * r, where r is
 the hardware reciprocal of s (within 1 ulp of 1/s), and falls back to the
 IEEE division when y lies within 4e-5 of a half-integer.  The reference
