@@ -781,4 +781,68 @@ pa_status_t pa_reshape_and_cache_f16(const void* key, const void* value,
   return pa::launch_cache_write_f16(l) == hipSuccess ? PA_OK : PA_ERR_LAUNCH;
 }
 
+size_t pa_cache_prefill_workspace_bytes(void) { return pa::kAmaxPartials * sizeof(uint32_t); }
+
+pa_status_t pa_cache_prefill(pa_cache_mode_t mode, int32_t bf16_input, const void* key,
+                             const void* value, int64_t key_token_stride, int64_t key_head_stride,
+                             int64_t value_token_stride, int64_t value_head_stride,
+                             const int64_t* slot_mapping, int32_t num_tokens, int32_t pad_tokens,
+                             int32_t num_kv_heads, int32_t head_dim, void* k_cache, void* v_cache,
+                             float* k_scales, float* v_scales, float* k_scale, float* v_scale,
+                             int32_t num_blocks, int32_t block_size, int32_t x, void* counters,
+                             size_t counter_bytes, void* workspace, size_t workspace_bytes,
+                             pa_stream_t stream) {
+  if (mode < PA_CACHE_F16 || mode > PA_CACHE_I8_TENSOR) return PA_ERR_BAD_SHAPE;
+  const bool int8 = mode != PA_CACHE_F16;
+  const pa_status_t st = check_write_args(
+      key, value, key_token_stride, key_head_stride, value_token_stride, value_head_stride,
+      slot_mapping, num_tokens, num_kv_heads, head_dim, k_cache, v_cache, num_blocks, block_size,
+      x, int8 ? 16 : 8);
+  if (st != PA_OK) return st;
+  if (pad_tokens < 0 || (!int8 && bf16_input) || (long long)num_tokens + pad_tokens > INT32_MAX)
+    return PA_ERR_BAD_SHAPE;
+  if (num_tokens == 0) return PA_OK;
+  if (int8 && (!k_scales || !v_scales)) return PA_ERR_NULL_POINTER;
+  pa::WriteLaunch l{};
+  l.key = key;
+  l.value = value;
+  l.key_token_stride = key_token_stride;
+  l.key_head_stride = key_head_stride;
+  l.value_token_stride = value_token_stride;
+  l.value_head_stride = value_head_stride;
+  l.slot_mapping = slot_mapping;
+  l.num_tokens = num_tokens;
+  l.pad_tokens = pad_tokens;
+  l.num_kv_heads = num_kv_heads;
+  l.head_dim = head_dim;
+  l.k_cache = k_cache;
+  l.v_cache = v_cache;
+  l.k_scales = k_scales;
+  l.v_scales = v_scales;
+  l.num_blocks = num_blocks;
+  l.block_size = block_size;
+  l.stream = reinterpret_cast<hipStream_t>(stream);
+  hipError_t e;
+  if (mode == PA_CACHE_F16) {
+    e = pa::launch_cache_write_f16(l);
+  } else if (mode == PA_CACHE_I8_TOKEN) {
+    e = bf16_input ? pa::launch_quant_write_i8<0, 1>(l) : pa::launch_quant_write_i8<0, 0>(l);
+  } else {
+    if (!k_scale || !v_scale) return PA_ERR_NULL_POINTER;
+    if (!counters || counter_bytes < pa::kAmaxCounterBytes || !workspace ||
+        workspace_bytes < pa_cache_prefill_workspace_bytes() ||
+        reinterpret_cast<uintptr_t>(counters) % 4 != 0 ||
+        reinterpret_cast<uintptr_t>(workspace) % 4 != 0)
+      return PA_ERR_WORKSPACE;
+    e = pa::launch_tensor_scales(l, bf16_input != 0, k_scale, v_scale,
+                                 static_cast<uint32_t*>(counters),
+                                 static_cast<uint32_t*>(workspace));
+    if (e != hipSuccess) return PA_ERR_LAUNCH;
+    l.k_scale_in = k_scale;
+    l.v_scale_in = v_scale;
+    e = bf16_input ? pa::launch_quant_write_i8<1, 1>(l) : pa::launch_quant_write_i8<1, 0>(l);
+  }
+  return e == hipSuccess ? PA_OK : PA_ERR_LAUNCH;
+}
+
 }  // extern "C"

@@ -162,6 +162,7 @@ struct WriteLaunch {
   int64_t value_head_stride;
   const int64_t* slot_mapping;
   int num_tokens;
+  int pad_tokens;    // slots after the tokens', written as zeros (needs num_tokens >= 1)
   int num_kv_heads;
   int head_dim;
   void* k_cache;
@@ -187,5 +188,13 @@ template <> hipError_t launch_quant_write_i8<0, 1>(const WriteLaunch& l);
 template <> hipError_t launch_quant_write_i8<1, 0>(const WriteLaunch& l);
 template <> hipError_t launch_quant_write_i8<1, 1>(const WriteLaunch& l);
 hipError_t launch_cache_write_f16(const WriteLaunch& l);
+
+// Per-tensor scales of a write's rows into *k_scale and *v_scale (pa_amax.hip).
+// `counter`: kAmaxCounterBytes, zero before and after; `partials`: kAmaxPartials words.
+constexpr int kAmaxGroups = 128;   // work-groups per tensor, at most
+constexpr int kAmaxPartials = 2 * kAmaxGroups;
+constexpr size_t kAmaxCounterBytes = (kSchedQueueStride + 1) * sizeof(uint32_t);
+hipError_t launch_tensor_scales(const WriteLaunch& l, bool bf16, float* k_scale, float* v_scale,
+                                uint32_t* counter, uint32_t* partials);
 
 }  // namespace pa

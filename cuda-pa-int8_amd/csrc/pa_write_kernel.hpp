@@ -213,7 +213,8 @@ struct WriteArgs {
   const uint16_t* value;
   int64_t kts, khs, vts, vhs;   // element strides of a token and of a head
   const int64_t* slots;         // num_tokens entries
-  int num_tokens;
+  int num_tokens;               // tokens with a slot
+  int num_rows;                 // of them, tokens with an input row (>= 1); the rest are zeros
   int hkv;
   void* kc;
   void* vc;
@@ -453,7 +454,7 @@ __device__ __forceinline__ Window find_runs(const WriteArgs& a, int t0, int lane
 template <int D>
 __device__ __forceinline__ void load_row(const WriteArgs& a, bool v, int h, int tb, int i, int qq,
                                          WriteRow<D>& r) {
-  const int64_t tok = min(tb + i, a.num_tokens - 1);
+  const int64_t tok = min(tb + i, a.num_rows - 1);
   const uint16_t* src = v ? a.value + tok * a.vts + (int64_t)h * a.vhs
                           : a.key + tok * a.kts + (int64_t)h * a.khs;
 #pragma unroll
@@ -473,6 +474,7 @@ __device__ __forceinline__ void write_run(const WriteArgs& a,
   const int bs = a.bs;
   const int64_t bh = (slot >> a.bs_log2) * a.hkv + h;
   const int off = (int)(slot & (bs - 1));
+  const bool pad = tb + ln.i >= a.num_rows;
   const RowScale q = row_scale<D, MODE, BF, PROBE>(r, v ? a.v_scale_in : a.k_scale_in);
   const uint32_t tile_bytes = (uint32_t)(D * bs * ESZ);
   const auto tile =
@@ -483,13 +485,14 @@ __device__ __forceinline__ void write_run(const WriteArgs& a,
     const int o = ln.qq + 4 * j;           // dim group: dims 8o .. 8o + 7
     if (o >= WriteRow<D>::DG) continue;    // padding group (whole 16-lane rows): nothing to write
     WriteGroup<MODE> g = row_group<MODE, BF, PROBE>(r.x[j], q);
+    if (pad) g = WriteGroup<MODE>{};
     if (!v) store_tile<kStoreStream>(tile, (o * bs + off + ln.i) * 8 * ESZ, g);
     else if (bs == 16) store_tile<kStoreStream>(tile, at_v(o), transpose_v(g, ln.ts));
     else store_tile<kStorePlain>(tile, at_v(o), transpose_v(g, ln.ts));
     __builtin_amdgcn_sched_barrier(0);
   }
   if constexpr (I8) {
-    if (ln.qq == 0) (v ? a.vsc : a.ksc)[bh * bs + off + ln.i] = q.s;
+    if (ln.qq == 0) (v ? a.vsc : a.ksc)[bh * bs + off + ln.i] = pad ? 0.f : q.s;
   }
 }
 
@@ -505,12 +508,16 @@ __device__ __forceinline__ void write_loose(const WriteArgs& a,
   using Group = WriteGroup<MODE>;
   const int bs = a.bs;
   const bool mine = (loose >> ln.i) & 1;
+  const bool pad = t0 + ln.i >= a.num_rows;
   const int64_t bh = (mine ? sl >> a.bs_log2 : 0) * a.hkv + h;
   const int off = mine ? (int)(sl & (bs - 1)) : 0;
   const RowScale q = row_scale<D, MODE, BF, PROBE>(r, v ? a.v_scale_in : a.k_scale_in);
   Group g[JQ];
 #pragma unroll
-  for (int j = 0; j < JQ; ++j) g[j] = row_group<MODE, BF, PROBE>(r.x[j], q);
+  for (int j = 0; j < JQ; ++j) {
+    g[j] = row_group<MODE, BF, PROBE>(r.x[j], q);
+    if (pad) g[j] = Group{};
+  }
   if (!v) {
     uint8_t* const dst = static_cast<uint8_t*>(a.kc) + (bh * DG * bs + off) * 8 * ESZ;
     if (mine) {
@@ -545,7 +552,7 @@ __device__ __forceinline__ void write_loose(const WriteArgs& a,
     }
   }
   if constexpr (I8) {
-    if (ln.qq == 0 && mine) (v ? a.vsc : a.ksc)[bh * bs + off] = q.s;
+    if (ln.qq == 0 && mine) (v ? a.vsc : a.ksc)[bh * bs + off] = pad ? 0.f : q.s;
   }
 }
 
@@ -637,7 +644,8 @@ hipError_t launch_write(const WriteLaunch& l) {
   a.vts = l.value_token_stride;
   a.vhs = l.value_head_stride;
   a.slots = l.slot_mapping;
-  a.num_tokens = l.num_tokens;
+  a.num_tokens = l.num_tokens + l.pad_tokens;
+  a.num_rows = l.num_tokens;
   a.hkv = l.num_kv_heads;
   a.kc = l.k_cache;
   a.vc = l.v_cache;
@@ -648,7 +656,7 @@ hipError_t launch_write(const WriteLaunch& l) {
   a.bs = l.block_size;
   a.bs_log2 = __builtin_ctz((unsigned)l.block_size);
   a.pool = (int64_t)l.num_blocks * l.block_size;
-  const long long windows = (l.num_tokens + 15ll) / 16;
+  const long long windows = (a.num_tokens + 15ll) / 16;
   const long long small = 4 * windows * l.num_kv_heads;
   if (small <= kSmallWaves) {
     const int nw = small <= kSmallSpreadWaves ? 1 : kWriteWaves;

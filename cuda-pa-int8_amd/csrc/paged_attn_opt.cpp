@@ -296,7 +296,8 @@ std::pair<int64_t, int64_t> decode_plan(int64_t kind, int64_t num_seqs, int64_t 
 // whether scale tensors are passed.
 void check_write(const at::Tensor& key, const at::Tensor& value, const at::Tensor& k_cache,
                  const at::Tensor& v_cache, const at::Tensor* k_scales,
-                 const at::Tensor* v_scales, const at::Tensor& slot_mapping, bool int8) {
+                 const at::Tensor* v_scales, const at::Tensor& slot_mapping, bool int8,
+                 int64_t pad_tokens = 0) {
   TORCH_CHECK(key.is_cuda() && value.is_cuda(), "tensors must be on CUDA");
   if (int8) {
     TORCH_CHECK((key.scalar_type() == at::kHalf || key.scalar_type() == at::kBFloat16) &&
@@ -325,7 +326,7 @@ void check_write(const at::Tensor& key, const at::Tensor& value, const at::Tenso
   TORCH_CHECK(k_cache.size(1) == Hkv && k_cache.size(2) * x == D && v_cache.size(0) == NB &&
                   v_cache.size(1) == Hkv && v_cache.size(2) == D && v_cache.size(3) == bs,
               "cache shapes do not match key/value");
-  TORCH_CHECK(slot_mapping.dim() == 1 && slot_mapping.size(0) == T,
+  TORCH_CHECK(slot_mapping.dim() == 1 && slot_mapping.size(0) == T + pad_tokens,
               "slot_mapping must be [num_tokens]");
   for (const at::Tensor* t : {&k_cache, &v_cache, &slot_mapping})
     TORCH_CHECK(t->is_contiguous() && t->is_cuda() && t->get_device() == key.get_device(),
@@ -395,6 +396,47 @@ void reshape_and_cache(at::Tensor key, at::Tensor value, at::Tensor k_cache, at:
       reinterpret_cast<pa_stream_t>(stream)));
 }
 
+// NEW op: one layer's prompt write (PagedKVCache.prefill): the rows at the first
+// slots of slot_mapping, zeros in the slots that follow.  `tensor_scales`
+// (INT8): the two per-tensor scales, taken from the rows and written here;
+// without them the INT8 scales are per token.
+void cache_prefill(at::Tensor key, at::Tensor value, at::Tensor k_cache, at::Tensor v_cache,
+                   c10::optional<at::Tensor> k_scales, c10::optional<at::Tensor> v_scales,
+                   at::Tensor slot_mapping, c10::optional<at::Tensor> tensor_scales) {
+  const bool int8 = k_scales.has_value();
+  TORCH_CHECK(int8 == v_scales.has_value() && (int8 || !tensor_scales.has_value()),
+              "scales go with INT8 caches");
+  TORCH_CHECK(key.dim() == 3 && slot_mapping.dim() == 1 && slot_mapping.size(0) >= key.size(0),
+              "slot_mapping must hold a slot for every token");
+  const int64_t pad = slot_mapping.size(0) - key.size(0);
+  check_write(key, value, k_cache, v_cache, int8 ? &*k_scales : nullptr,
+              int8 ? &*v_scales : nullptr, slot_mapping, int8, pad);
+  const at::hip::HIPGuardMasqueradingAsCUDA guard(key.device());
+  hipStream_t stream = at::hip::getCurrentHIPStreamMasqueradingAsCUDA(key.get_device()).stream();
+  pa_cache_mode_t mode = int8 ? PA_CACHE_I8_TOKEN : PA_CACHE_F16;
+  float* ts = nullptr;
+  at::Tensor cnt, ws;
+  if (tensor_scales.has_value()) {
+    const at::Tensor& t = *tensor_scales;
+    TORCH_CHECK(t.numel() == 2 && t.scalar_type() == at::kFloat && t.is_contiguous() &&
+                    t.is_cuda() && t.get_device() == key.get_device(),
+                "tensor_scales must be two fp32 values on key's device");
+    mode = PA_CACHE_I8_TENSOR;
+    ts = t.data_ptr<float>();
+    cnt = counters_for(key, stream, kMinCounterBytes);
+    ws = at::empty({(int64_t)pa_cache_prefill_workspace_bytes()}, key.options().dtype(at::kByte));
+  }
+  check_status(pa_cache_prefill(
+      mode, key.scalar_type() == at::kBFloat16, key.data_ptr(), value.data_ptr(), key.stride(0),
+      key.stride(1), value.stride(0), value.stride(1), slot_mapping.data_ptr<int64_t>(),
+      (int32_t)key.size(0), (int32_t)pad, (int32_t)key.size(1), (int32_t)key.size(2),
+      k_cache.data_ptr(), v_cache.data_ptr(), int8 ? k_scales->data_ptr<float>() : nullptr,
+      int8 ? v_scales->data_ptr<float>() : nullptr, ts, ts ? ts + 1 : nullptr,
+      (int32_t)k_cache.size(0), (int32_t)k_cache.size(3), (int32_t)k_cache.size(4),
+      ts ? cnt.data_ptr() : nullptr, ts ? (size_t)cnt.numel() : 0, ts ? ws.data_ptr() : nullptr,
+      ts ? (size_t)ws.numel() : 0, reinterpret_cast<pa_stream_t>(stream)));
+}
+
 }  // namespace
 
 PYBIND11_MODULE(paged_attn_opt, m) {
@@ -422,6 +464,9 @@ PYBIND11_MODULE(paged_attn_opt, m) {
   m.def("reshape_and_cache_int8_static", &reshape_and_cache_int8_static,
         "INT8 quantize with one given scale per K / V tensor + paged cache write (new op)");
   m.def("reshape_and_cache", &reshape_and_cache, "fp16 paged cache write (new op)");
+  m.def("cache_prefill", &cache_prefill,
+        "one prompt's cache write with the rest of its last block zeroed; per-tensor scales "
+        "taken from the rows when asked for (new op)");
   m.def("version", []() { return std::string(pa_version()); });
 }
 

@@ -39,6 +39,7 @@ PROBE_LIB_NAME = "libpa_bench_probe.so"
 HEAD_DIMS = tuple(range(8, 257, 8))
 HIP_SOURCES = [
     "pa_cache_write.hip",
+    "pa_amax.hip",
     "pa_fill.hip",
     "pa_noalloc.hip",
 ]

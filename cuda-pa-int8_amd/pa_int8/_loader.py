@@ -109,6 +109,10 @@ PROTOTYPES = {
     "pa_reshape_and_cache_int8_static_bf16": (ctypes.c_int, [_p, _p, _i64, _i64, _i64, _i64, _p,
                                                              _i32, _i32, _i32, _p, _p, _p, _p, _p,
                                                              _p, _i32, _i32, _i32, _p]),
+    "pa_cache_prefill_workspace_bytes": (_sz, []),
+    "pa_cache_prefill": (ctypes.c_int, [ctypes.c_int, _i32, _p, _p, _i64, _i64, _i64, _i64, _p, _i32,
+                                        _i32, _i32, _i32, _p, _p, _p, _p, _p, _p, _i32, _i32, _i32,
+                                        _p, _sz, _p, _sz, _p]),
     "pa_reshape_and_cache_f16": (ctypes.c_int, [_p, _p, _i64, _i64, _i64, _i64, _p, _i32, _i32,
                                                 _i32, _p, _p, _i32, _i32, _i32, _p]),
 }

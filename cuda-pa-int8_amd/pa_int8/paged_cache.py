@@ -16,9 +16,10 @@ layouts).  The three variants are the reference's:
   (write: ``reshape_and_cache_int8_static``).
 
 Where the reference quantizes with several torch ops and scatters with
-permuted copies, each write here is one kernel launch; the per-tensor amax
-is a torch reduction on the device.  ``prefill`` also clears the unused tail
-of the last block, as the reference's zero-padded copy does (:116-128).
+permuted copies, each write here is one kernel launch, and a per-tensor prefill
+two: its scales, then the write.  ``prefill`` also clears the unused tail
+of the last block, as the reference's zero-padded copy does (:116-128), in the
+same launch.
 Writes take fp16 K/V on a HIP device, and the INT8 variants bf16 too (the
 dtype the reference's bridge runs Qwen in, quantized directly as its
 quantize_per_token does); the fp16 variant converts other float dtypes first,
@@ -146,20 +147,21 @@ class PagedKVCache:
         assert H == self.num_kv_heads and D == self.head_dim
         assert L <= self.num_blocks * self.block_size
         k, v = self._kernel_input(k), self._kernel_input(v)
+        scales = None
         if self.variant == "int8_per_tensor":
-            self._k_tensor_scale[layer_idx] = (
-                (k.abs().amax() / 127.0).to(torch.float32).clamp_min(1e-8).reshape(1))
-            self._v_tensor_scale[layer_idx] = (
-                (v.abs().amax() / 127.0).to(torch.float32).clamp_min(1e-8).reshape(1))
+            if L == 0:
+                raise RuntimeError("int8_per_tensor: the scales of an empty prompt are undefined")
+            scales = torch.empty(2, dtype=torch.float32, device=k.device)
         if L > 0:
-            self._write(layer_idx, k, v, self._slots[:L])
-        # the rest of the last block holds zeros, as after the reference's padded copy
-        off = L % self.block_size
-        if off:
-            blk = L // self.block_size
-            for name, (_, _, tok_axis) in self.layout.tensors().items():
-                getattr(self, name)[layer_idx, blk].narrow(tok_axis, off,
-                                                           self.block_size - off).zero_()
+            # The rest of the last block holds zeros, as after the reference's padded copy.
+            slots = self._slots[:self.layout.blocks_for(L) * self.block_size]
+            ks, vs = ((self.k_scales[layer_idx], self.v_scales[layer_idx]) if self.is_int8
+                      else (None, None))
+            registry.cache_prefill(k, v, self.k_cache[layer_idx], self.v_cache[layer_idx], ks, vs,
+                                   slots, scales)
+        if scales is not None:
+            self._k_tensor_scale[layer_idx] = scales[:1]
+            self._v_tensor_scale[layer_idx] = scales[1:]
         self.lengths[layer_idx] = L
 
     def decode_append(self, layer_idx, k, v):

@@ -109,3 +109,14 @@ def reshape_and_cache(key, value, k_cache, v_cache, slot_mapping):
     """fp16 write of ``key/value [T, Hkv, D]`` into the paged fp16 cache at
     ``slot_mapping`` (the fp16 mode of PagedKVCache, paged_cache.py:116-130,148-150)."""
     _ext().reshape_and_cache(key, value, k_cache, v_cache, slot_mapping)
+
+
+def cache_prefill(key, value, k_cache, v_cache, k_scales, v_scales, slot_mapping,
+                  tensor_scales=None):
+    """One prompt's write: ``key/value [T, Hkv, D]`` at the first T slots of
+    ``slot_mapping`` and zeros at the slots that follow.  fp16 without scales, INT8
+    with per-token scales, or, given ``tensor_scales`` (two fp32 on the device,
+    written here), with one scale per tensor taken from the rows (the three
+    modes of PagedKVCache.prefill, benchmarks/int8_bridge/paged_cache.py:88-130)."""
+    _ext().cache_prefill(key, value, k_cache, v_cache, k_scales, v_scales, slot_mapping,
+                         tensor_scales)

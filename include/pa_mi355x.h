@@ -264,6 +264,35 @@ pa_status_t pa_reshape_and_cache_f16(
     void* k_cache, void* v_cache, int32_t num_blocks, int32_t block_size, int32_t x,
     pa_stream_t stream);
 
+/* One layer's prompt write of PagedKVCache (benchmarks/int8_bridge/paged_cache.py:88-130)
+ * without per-op passes.  NEW API: the write of `mode` above for num_tokens rows at
+ * slot_mapping[0 .. num_tokens), and zeros (values and scales) in the pad_tokens
+ * slots that follow in slot_mapping: the rest of the prompt's last block, which
+ * the reference's padded copy leaves zero (:116-128).  PA_CACHE_I8_TENSOR first takes
+ * the per-tensor scales from the rows (:101-102, max(fp32(t(amax / 127)), 1e-8) with t
+ * the input type) and leaves them in *k_scale and *v_scale (device); it needs
+ * `counters` (256 bytes or more, zero before and after the call, shared with other calls
+ * under the rules of the decode counters) and a workspace of
+ * pa_cache_prefill_workspace_bytes(); the other modes ignore these four and the
+ * scale pointers.  bf16_input: the rows are bf16 (INT8 modes only).  With
+ * num_tokens = 0 nothing is written.  Other rules as pa_reshape_and_cache_int8 /
+ * _f16. */
+typedef enum pa_cache_mode {
+  PA_CACHE_F16 = 0,
+  PA_CACHE_I8_TOKEN = 1,
+  PA_CACHE_I8_TENSOR = 2
+} pa_cache_mode_t;
+size_t pa_cache_prefill_workspace_bytes(void);
+pa_status_t pa_cache_prefill(pa_cache_mode_t mode, int32_t bf16_input, const void* key,
+                             const void* value, int64_t key_token_stride, int64_t key_head_stride,
+                             int64_t value_token_stride, int64_t value_head_stride,
+                             const int64_t* slot_mapping, int32_t num_tokens, int32_t pad_tokens,
+                             int32_t num_kv_heads, int32_t head_dim, void* k_cache, void* v_cache,
+                             float* k_scales, float* v_scales, float* k_scale, float* v_scale,
+                             int32_t num_blocks, int32_t block_size, int32_t x, void* counters,
+                             size_t counter_bytes, void* workspace, size_t workspace_bytes,
+                             pa_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif
