@@ -500,6 +500,16 @@ pa_status_t pa_check_context_lens(const int32_t* host_context_lens, int32_t num_
   return PA_OK;
 }
 
+pa_status_t pa_context_lens_range(const int32_t* context_lens, int32_t num_seqs, uint64_t* out,
+                                  uint32_t tag, pa_stream_t stream) {
+  if (!context_lens || !out) return PA_ERR_NULL_POINTER;
+  if (num_seqs < 1) return PA_ERR_BAD_SHAPE;
+  return pa::launch_ctx_range(context_lens, num_seqs, out, tag,
+                              reinterpret_cast<hipStream_t>(stream)) == hipSuccess
+             ? PA_OK
+             : PA_ERR_LAUNCH;
+}
+
 pa_status_t pa_decode_plan(pa_decode_kind_t kind, int32_t num_seqs, int32_t num_heads,
                            int32_t head_dim, int32_t num_kv_heads, int32_t block_size,
                            int32_t max_blocks_per_seq, int32_t max_context_len,

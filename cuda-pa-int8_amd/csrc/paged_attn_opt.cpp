@@ -7,6 +7,8 @@
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 
+#include <atomic>
+#include <chrono>
 #include <map>
 #include <mutex>
 #include <utility>
@@ -70,6 +72,79 @@ at::Tensor counters_for(const at::Tensor& like, hipStream_t stream, size_t bytes
 
 void check_status(pa_status_t st) { TORCH_CHECK(st == PA_OK, pa_status_string(st)); }
 
+// Result slots of the context-length check: coherent host memory that a kernel
+// writes and the host polls.  One 4 KB block for the process, kept until it ends
+// (the driver may still be mapping it when a thread ends); a call holds one slot
+// until its kernel has written it, and finding none free is no error.
+struct RangeSlots {
+  static constexpr int kSlots = 32;
+  uint64_t* mem = nullptr;                  // kSlots x 8 words (a line each)
+  std::atomic<uint32_t> taken{0};
+  std::atomic<uint32_t> tag{0};
+  RangeSlots() {
+    void* p = nullptr;
+    if (hipHostMalloc(&p, 4096, hipHostMallocCoherent | hipHostMallocMapped |
+                                    hipHostMallocPortable) == hipSuccess)
+      mem = static_cast<uint64_t*>(p);
+    else
+      (void)hipGetLastError();
+  }
+  int take() {
+    uint32_t t = taken.load();
+    while (mem != nullptr && t != 0xFFFFFFFFu) {
+      const int i = __builtin_ctz(~t);
+      if (taken.compare_exchange_weak(t, t | (1u << i))) return i;
+    }
+    return -1;
+  }
+  void give(int i) { taken.fetch_and(~(1u << i)); }
+};
+
+// Smallest and largest context length through a kernel that writes them where the
+// host polls.  False (nothing done) where that does not apply: lengths elsewhere
+// than on q's device or not dense (a later check reports them), a stream under
+// capture, no free slot.
+bool polled_range(const at::Tensor& ctx, const at::Tensor& q, int32_t* mn, int32_t* mx) {
+  if (!ctx.is_cuda() || ctx.get_device() != q.get_device() || !ctx.is_contiguous() ||
+      ctx.numel() > INT32_MAX)
+    return false;
+  const at::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
+  hipStream_t stream = at::hip::getCurrentHIPStreamMasqueradingAsCUDA(q.get_device()).stream();
+  if (stream_capturing(stream)) return false;
+  static RangeSlots* slots = new RangeSlots();
+  const int i = slots->take();
+  if (i < 0) return false;
+  volatile uint64_t* w = slots->mem + 8 * i;
+  const uint32_t tag = slots->tag.fetch_add(1) + 1;
+  w[0] = w[1] = (uint64_t)(tag - 1) << 32;   // whatever the slot holds is not this call's tag
+  std::atomic_thread_fence(std::memory_order_seq_cst);
+  const pa_status_t st =
+      pa_context_lens_range(ctx.data_ptr<int32_t>(), (int32_t)ctx.numel(), slots->mem + 8 * i, tag,
+                            reinterpret_cast<pa_stream_t>(stream));
+  if (st != PA_OK) {
+    slots->give(i);
+    check_status(st);
+  }
+  // The stream may have other work before the kernel: poll for about as long as
+  // a blocked wait costs more than it saves, then wait on the stream.
+  const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(1);
+  auto done = [&] { return (uint32_t)(w[0] >> 32) == tag && (uint32_t)(w[1] >> 32) == tag; };
+  for (int spin = 0; !done(); ++spin) {
+    __builtin_ia32_pause();
+    if ((spin & 63) == 63 && std::chrono::steady_clock::now() > until) {
+      const hipError_t e = hipStreamSynchronize(stream);
+      // (after a failed wait the kernel's fate is unknown: its slot stays taken)
+      TORCH_CHECK(e == hipSuccess, "context_lens check: ", hipGetErrorString(e));
+      TORCH_CHECK(done(), "context_lens check: the kernel's result did not arrive");
+    }
+  }
+  *mn = (int32_t)(uint32_t)w[0];
+  *mx = (int32_t)(uint32_t)w[1];
+  slots->give(i);
+  return true;
+}
+
+
 // Which reference launcher's block_size rule an op repeats: the naive stage
 // checks none (paged_attention_naive.cu:135-140), the vectorised stage only a
 // multiple of 8 (paged_attention_v1_vectorized.cu:124), the later ones also
@@ -102,12 +177,15 @@ void run_decode(pa_decode_kind_t kind, at::Tensor& out, const at::Tensor& q,
   int32_t max_ctx = 0;
   bool equal_lens = false;
   if (check_context && context_lens.numel() > 0) {
-    // One device->host copy for both the reference's `min >= 1` rule
-    // (v3:147-148) and the split count (v4:213-214).
-    const auto mnmx = at::aminmax(context_lens);
-    const at::Tensor mm = at::stack({std::get<0>(mnmx), std::get<1>(mnmx)}).cpu();
-    const int32_t mn = mm[0].item<int32_t>();
-    max_ctx = mm[1].item<int32_t>();
+    // One read-back for both the reference's `min >= 1` rule (v3:147-148) and the
+    // split count (v4:213-214).
+    int32_t mn = 0;
+    if (!polled_range(context_lens, q, &mn, &max_ctx)) {
+      const auto mnmx = at::aminmax(context_lens);
+      const at::Tensor mm = at::stack({std::get<0>(mnmx), std::get<1>(mnmx)}).cpu();
+      mn = mm[0].item<int32_t>();
+      max_ctx = mm[1].item<int32_t>();
+    }
     TORCH_CHECK(mn >= 1, "context_lens must be >= 1 (empty sequences unsupported)");
     equal_lens = mn == max_ctx;
   }

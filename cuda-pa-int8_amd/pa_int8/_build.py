@@ -40,6 +40,7 @@ HEAD_DIMS = tuple(range(8, 257, 8))
 HIP_SOURCES = [
     "pa_cache_write.hip",
     "pa_amax.hip",
+    "pa_ctx_range.hip",
     "pa_fill.hip",
     "pa_noalloc.hip",
 ]

@@ -109,6 +109,7 @@ PROTOTYPES = {
     "pa_reshape_and_cache_int8_static_bf16": (ctypes.c_int, [_p, _p, _i64, _i64, _i64, _i64, _p,
                                                              _i32, _i32, _i32, _p, _p, _p, _p, _p,
                                                              _p, _i32, _i32, _i32, _p]),
+    "pa_context_lens_range": (ctypes.c_int, [_p, _i32, _p, ctypes.c_uint32, _p]),
     "pa_cache_prefill_workspace_bytes": (_sz, []),
     "pa_cache_prefill": (ctypes.c_int, [ctypes.c_int, _i32, _p, _p, _i64, _i64, _i64, _i64, _p, _i32,
                                         _i32, _i32, _i32, _p, _p, _p, _p, _p, _p, _i32, _i32, _i32,

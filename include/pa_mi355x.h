@@ -92,6 +92,13 @@ pa_status_t pa_validate_decode(pa_decode_kind_t kind, int32_t num_seqs, int32_t 
 pa_status_t pa_check_context_lens(const int32_t* host_context_lens, int32_t num_seqs,
                                   int32_t* max_len);
 
+/* Range of context lengths on the device, for that check without a copy and a
+ * synchronization.  out[0] = tag << 32 | minimum and out[1] = tag << 32 | maximum, each
+ * word stored once, at system scope: with `out` in coherent host memory the caller polls
+ * both words for its tag.  num_seqs >= 1. */
+pa_status_t pa_context_lens_range(const int32_t* context_lens, int32_t num_seqs, uint64_t* out,
+                                  uint32_t tag, pa_stream_t stream);
+
 /* Split plan of the grid form: how many tokens each work-group covers (a
  * multiple of 64) and how many splits the longest sequence needs.  (Under the
  * in-kernel schedule the kernel picks the partition on the device from the

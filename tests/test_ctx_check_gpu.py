@@ -1,0 +1,105 @@
+"""GPU tests of the ops' context-length check (the reference's `min >= 1` rule,
+paged_attention_v3_warp.cu:147-148), whose result a kernel writes where the
+host polls: positions of the extremes, batches around the reduction's sizes,
+work queued before it, several streams and threads, and capture."""
+
+import threading
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _lib(built):
+    import pa_int8
+
+    pa_int8.ext()
+
+
+def inputs(n, cap=64, seed=0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    blocks = cap // 16
+    kc = torch.randn(n * blocks, 1, 1, 16, 8, device=DEV, generator=g).half()
+    vc = torch.randn(n * blocks, 1, 8, 16, device=DEV, generator=g).half()
+    bt = torch.arange(n * blocks, dtype=torch.int32, device=DEV).view(n, blocks)
+    q = torch.randn(n, 1, 8, device=DEV, generator=g).half()
+    ctx = torch.randint(1, cap + 1, (n,), device=DEV, generator=g).to(torch.int32)
+    return q, kc, vc, bt, ctx
+
+
+def call(x, variant="warp"):
+    import pa_int8
+
+    q, kc, vc, bt, ctx = x
+    out = torch.full_like(q, 7)
+    pa_int8.VARIANTS[variant](out, q, kc, vc, bt, ctx, 0.3, 16)
+    return out
+
+
+def unchecked(x, variant="warp"):
+    import pa_int8
+
+    q, kc, vc, bt, ctx = x
+    return pa_int8.decode(variant, torch.empty_like(q), q, kc, vc, bt, ctx, 0.3, 16, check=False)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 255, 256, 257, 1000])
+def test_extremes_are_found(n):
+    x = inputs(n)
+    torch.testing.assert_close(call(x), unchecked(x), rtol=0, atol=0)
+    for bad in (0, -5):
+        for at in {0, n // 2, n - 1}:
+            y = x[:4] + (x[4].clone(),)
+            y[4][at] = bad
+            out = torch.full_like(x[0], 7)
+            import pa_int8
+            with pytest.raises(RuntimeError, match="context_lens must be >= 1"):
+                pa_int8.VARIANTS["warp"](out, *y, 0.3, 16)
+            assert (out == 7).all()      # a refused call leaves its output alone
+    torch.testing.assert_close(call(x, "splitk"), unchecked(x, "splitk"), rtol=0, atol=1e-3)
+
+
+def test_behind_queued_work():
+    """The lengths are produced by work that is still queued (longer than the
+    check polls before it waits on the stream)."""
+    x = inputs(8)
+    a = torch.randn(4096, 4096, device=DEV)
+    for _ in range(60):
+        a = (a @ a) * 1e-3
+    late = (x[4].float() + 0 * a[0, 0].nan_to_num()).to(torch.int32)
+    torch.testing.assert_close(call(x[:4] + (late,)), unchecked(x), rtol=0, atol=0)
+
+
+def test_threads_and_streams():
+    cases = [inputs(3 + i, seed=i) for i in range(6)]
+    want = [unchecked(c) for c in cases]
+    torch.cuda.synchronize()
+    errors = []
+
+    def work(i):
+        try:
+            s = torch.cuda.Stream()
+            with torch.cuda.stream(s):
+                for _ in range(50):
+                    got = call(cases[i])
+                    s.synchronize()
+                    assert torch.equal(got, want[i])
+        except Exception as e:       # noqa: BLE001
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(6)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors[0]
+
+
+def test_non_contiguous_lengths_are_still_refused():
+    x = inputs(4)
+    wide = torch.stack([x[4], x[4]], dim=1)
+    with pytest.raises(RuntimeError, match="contiguous"):
+        call(x[:4] + (wide[:, 0],))
