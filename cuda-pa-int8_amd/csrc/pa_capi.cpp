@@ -42,10 +42,9 @@ int resident_groups(int head_dim, bool stream_part, int waves, bool int8_kv, int
 namespace {
 
 constexpr int kRefTile = 128;        // reference TILE (paged_attention_v3_warp.cu:20)
-// Split planning, from partition-size sweeps on MI355X (bench configs 2-4):
-// about 2048 resident waves (2 per SIMD with the pipelined loop) in as few
-// splits as possible gave the best times; smaller partitions pay more merge
-// round trips, larger ones leave CUs idle.
+// Split planning (pick_partition): about 2048 resident waves (2 per SIMD with the
+// pipelined loop) in as few splits as possible; smaller partitions pay more
+// merge round trips, larger ones leave CUs idle.
 constexpr int kTargetWaves = 2048;   // waves one decode launch aims for (256 CUs x 8)
 constexpr int kMinPartition = 256;   // per 4 waves: one 64-token iteration each
 // Shortest item of the in-kernel schedule on ragged lengths, in tokens at
@@ -116,6 +115,50 @@ struct Plan {
   bool k_nt = false;      // non-temporal K-row loads too
   bool fused = false;     // splits merged in the same launch (last-arriving work-group)
 };
+
+// Tokens per split of `units` units of `ctx` tokens (row_bytes of K/V each): a
+// multiple of `step` in [lo, hi].  What a launch costs, in tokens of a CU's time:
+// the rounds its work-groups take, one per CU at a time, times a split; no less than
+// the work spread over three quarters of the CUs, which already draw the full
+// bandwidth; a fixed cost per round (128 KB worth: block ids, first rows, epilogue)
+// and one for merging at all (200 KB).  Work-groups just past a whole round are the
+// expensive case: the CUs that hold two of them take twice as long, while the rest
+// of the chip is idle.  Candidates: per number of rounds, the most splits that fit and
+// the fewest that fill three quarters.  MI355X, fixed 256-work-group target ->
+// this rule, us (fp16 / INT8, head_dim 128): 17 x 21128 at 12/2 heads (34 units) 84.4 ->
+// 60 / 50.9 -> 36; 48 x 8192 12/2 87.8 -> 64.2 / 54.2 -> 39.4; 9 x 8192 32/8 66.2 ->
+// 51.0 / 41.7 -> 30.8; 70 x 2048 12/2 38.6 -> 28.4 / 24.3 -> 16.9; 36 x 3000 32/8 (288
+// units, more than a round unsplit) 88.4 -> 80.1 / 53.5 -> 47.1; head_dim 256: 12 x 6000 8/4
+// 55.6 -> 48.0 / 35.3 -> 31.3; the same plans where the units divide the CUs.
+long long pick_partition(long long ctx, long long units, long long lo, long long hi, long long step,
+                         long long row_bytes) {
+  const long long cus = kTargetWaves / 8;
+  const long long fill = (ctx * units * 4 + 3 * cus - 1) / (3 * cus);
+  const long long round_cost = (128 << 10) / row_bytes, merge_cost = (200 << 10) / row_bytes;
+  const long long n_min = (ctx + hi - 1) / hi, n_max = std::max(n_min, (ctx + lo - 1) / lo);
+  long long best = 0, best_cost = 0;
+  auto consider = [&](long long n) {
+    n = std::min(std::max(n, n_min), n_max);
+    long long part = ((ctx + n - 1) / n + step - 1) / step * step;
+    part = std::min(std::max(part, lo), hi);
+    n = (ctx + part - 1) / part;
+    const long long rounds = (units * n + cus - 1) / cus;
+    const long long cost =
+        std::max(rounds * part, fill) + rounds * round_cost + (n > 1 ? merge_cost : 0);
+    if (best == 0 || cost < best_cost) {
+      best = part;
+      best_cost = cost;
+    }
+  };
+  consider(n_min);
+  for (long long r = 1; r <= 4; ++r) {
+    const long long most = cus * r / units;
+    if (most < 1) continue;
+    consider(std::min(most, (cus * r * 3 / 4 + units - 1) / units));
+    consider(most);
+  }
+  return best;
+}
 
 Plan make_plan(pa_decode_kind_t kind, int num_seqs, int num_heads, int num_kv_heads,
                int head_dim, int block_size, int max_blocks, int max_context_len,
@@ -209,13 +252,12 @@ Plan make_plan(pa_decode_kind_t kind, int num_seqs, int num_heads, int num_kv_he
   if (partition_tokens > 0) {
     part = std::min<long long>(partition_tokens, hi);
   } else {
-    const long long units = std::max(1, p.units);
-    const int plan_waves = quad ? 8 : p.waves;   // the group size the split count assumes
-    const long long groups = kTargetWaves / plan_waves;
-    const long long lo = (long long)kMinPartition * plan_waves / 4;
-    part = (ctx * units + groups - 1) / groups;
-    part = (part + kMinPartition - 1) / kMinPartition * kMinPartition;
-    part = std::min(std::max(part, lo), hi);
+    const int plan_waves = quad ? 8 : p.waves;   // the group size the shortest split assumes
+    const long long lo = head_dim > 128 ? kMinPartition / 2
+                                        : (long long)kMinPartition * plan_waves / 4;
+    part = pick_partition(ctx, std::max(1, p.units), lo, hi,
+                          head_dim > 128 ? kMinPartition / 2 : kMinPartition,
+                          2ll * head_dim * (is_f16(kind) ? 2 : 1));
   }
   part = (part + pa::kIterTokens - 1) / pa::kIterTokens * pa::kIterTokens;
   part = std::min<long long>(part, (ctx + pa::kIterTokens - 1) / pa::kIterTokens * pa::kIterTokens);
