@@ -1,8 +1,8 @@
-// Smallest and largest context length of a batch, into memory the host polls (gfx950).
+// Smallest, largest and mean context length of a batch, into memory the host polls (gfx950).
 //
 // The reference's ops read context_lens.min() (and max()) back before every launch
 // (kernels/paged_attention_v3_warp.cu:147-148, v4_splitk.cu:213-214).  One small
-// launch reduces both and stores them, each in one 64-bit word with the caller's
+// launch reduces them and stores each in one 64-bit word with the caller's
 // tag, write-through to system memory: the host sees the words while the kernel
 // is still retiring and needs no copy and no stream synchronization.  Latency is
 // all there is to it: on MI355X a checked call over 4 short sequences takes 13.8 us
@@ -18,21 +18,26 @@ constexpr int kRangeThreads = 256;
 __global__ void __launch_bounds__(kRangeThreads)
 ctx_range_kernel(const int32_t* __restrict__ ctx, int n, uint64_t* out, uint32_t tag) {
   __shared__ int red[2][kRangeThreads / kWave];
+  __shared__ long long sums[kRangeThreads / kWave];
   int mn = INT32_MAX, mx = INT32_MIN;
+  long long sum = 0;
   for (int i = threadIdx.x; i < n; i += kRangeThreads) {
     const int v = ctx[i];
     mn = v < mn ? v : mn;
     mx = v > mx ? v : mx;
+    sum += v;
   }
 #pragma unroll
   for (int o = 1; o < kWave; o <<= 1) {
     const int a = __shfl_xor(mn, o, kWave), b = __shfl_xor(mx, o, kWave);
     mn = a < mn ? a : mn;
     mx = b > mx ? b : mx;
+    sum += __shfl_xor(sum, o, kWave);
   }
   if ((threadIdx.x & (kWave - 1)) == 0) {
     red[0][threadIdx.x >> 6] = mn;
     red[1][threadIdx.x >> 6] = mx;
+    sums[threadIdx.x >> 6] = sum;
   }
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -40,10 +45,13 @@ ctx_range_kernel(const int32_t* __restrict__ ctx, int n, uint64_t* out, uint32_t
     for (int i = 1; i < kRangeThreads / kWave; ++i) {
       mn = red[0][i] < mn ? red[0][i] : mn;
       mx = red[1][i] > mx ? red[1][i] : mx;
+      sum += sums[i];
     }
     const uint64_t t = (uint64_t)tag << 32;
     __hip_atomic_store(out, t | (uint32_t)mn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     __hip_atomic_store(out + 1, t | (uint32_t)mx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(out + 2, t | (uint32_t)(int)(sum / n), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 

@@ -151,7 +151,7 @@ PA_FOR_EACH_HEAD_DIM(PA_DECLARE_DECODE_D)
 // (pa_fill.hip).  A HIP graph may capture it: no memset node is recorded.
 hipError_t launch_fill_zero(void* p, size_t bytes, hipStream_t stream);
 
-// out[0] = tag << 32 | min, out[1] = tag << 32 | max of ctx[0 .. n) (pa_ctx_range.hip).
+// out[0 .. 2] = tag << 32 | the minimum, maximum and mean of ctx[0 .. n) (pa_ctx_range.hip).
 hipError_t launch_ctx_range(const int32_t* ctx, int n, uint64_t* out, uint32_t tag,
                             hipStream_t stream);
 

@@ -19,6 +19,7 @@
 namespace {
 
 constexpr int64_t kRefTile = 128;
+constexpr int32_t kMaxScheduledSeqs = 1024;   // batches the in-kernel schedule takes
 
 // Device memory of a decode call (include/pa_mi355x.h):
 //
@@ -100,11 +101,12 @@ struct RangeSlots {
   void give(int i) { taken.fetch_and(~(1u << i)); }
 };
 
-// Smallest and largest context length through a kernel that writes them where the
+// Smallest, largest and mean context length through a kernel that writes them where the
 // host polls.  False (nothing done) where that does not apply: lengths elsewhere
 // than on q's device or not dense (a later check reports them), a stream under
 // capture, no free slot.
-bool polled_range(const at::Tensor& ctx, const at::Tensor& q, int32_t* mn, int32_t* mx) {
+bool polled_range(const at::Tensor& ctx, const at::Tensor& q, int32_t* mn, int32_t* mx,
+                  int32_t* mean) {
   if (!ctx.is_cuda() || ctx.get_device() != q.get_device() || !ctx.is_contiguous() ||
       ctx.numel() > INT32_MAX)
     return false;
@@ -116,7 +118,7 @@ bool polled_range(const at::Tensor& ctx, const at::Tensor& q, int32_t* mn, int32
   if (i < 0) return false;
   volatile uint64_t* w = slots->mem + 8 * i;
   const uint32_t tag = slots->tag.fetch_add(1) + 1;
-  w[0] = w[1] = (uint64_t)(tag - 1) << 32;   // whatever the slot holds is not this call's tag
+  w[0] = w[1] = w[2] = (uint64_t)(tag - 1) << 32;   // whatever the slot holds is not this call's tag
   std::atomic_thread_fence(std::memory_order_seq_cst);
   const pa_status_t st =
       pa_context_lens_range(ctx.data_ptr<int32_t>(), (int32_t)ctx.numel(), slots->mem + 8 * i, tag,
@@ -128,7 +130,10 @@ bool polled_range(const at::Tensor& ctx, const at::Tensor& q, int32_t* mn, int32
   // The stream may have other work before the kernel: poll for about as long as
   // a blocked wait costs more than it saves, then wait on the stream.
   const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(1);
-  auto done = [&] { return (uint32_t)(w[0] >> 32) == tag && (uint32_t)(w[1] >> 32) == tag; };
+  auto done = [&] {
+    return (uint32_t)(w[0] >> 32) == tag && (uint32_t)(w[1] >> 32) == tag &&
+           (uint32_t)(w[2] >> 32) == tag;
+  };
   for (int spin = 0; !done(); ++spin) {
     __builtin_ia32_pause();
     if ((spin & 63) == 63 && std::chrono::steady_clock::now() > until) {
@@ -140,6 +145,7 @@ bool polled_range(const at::Tensor& ctx, const at::Tensor& q, int32_t* mn, int32
   }
   *mn = (int32_t)(uint32_t)w[0];
   *mx = (int32_t)(uint32_t)w[1];
+  *mean = (int32_t)(uint32_t)w[2];
   slots->give(i);
   return true;
 }
@@ -175,19 +181,21 @@ void run_decode(pa_decode_kind_t kind, at::Tensor& out, const at::Tensor& q,
   TORCH_CHECK(block_table.scalar_type() == at::kInt, "block_table must be int32");
   TORCH_CHECK(context_lens.scalar_type() == at::kInt, "context_lens must be int32");
   int32_t max_ctx = 0;
-  bool equal_lens = false;
+  int32_t mean_ctx = 0;   // 0: not known
   if (check_context && context_lens.numel() > 0) {
     // One read-back for both the reference's `min >= 1` rule (v3:147-148) and the
     // split count (v4:213-214).
     int32_t mn = 0;
-    if (!polled_range(context_lens, q, &mn, &max_ctx)) {
+    if (polled_range(context_lens, q, &mn, &max_ctx, &mean_ctx)) {
+      if (mn != max_ctx && mean_ctx == max_ctx) mean_ctx = max_ctx - 1;   // (equal means equal)
+    } else {
       const auto mnmx = at::aminmax(context_lens);
       const at::Tensor mm = at::stack({std::get<0>(mnmx), std::get<1>(mnmx)}).cpu();
       mn = mm[0].item<int32_t>();
       max_ctx = mm[1].item<int32_t>();
+      if (mn == max_ctx) mean_ctx = mn;
     }
     TORCH_CHECK(mn >= 1, "context_lens must be >= 1 (empty sequences unsupported)");
-    equal_lens = mn == max_ctx;
   }
   if (int8) {
     TORCH_CHECK(block_size % 16 == 0 && kRefTile % block_size == 0,
@@ -235,15 +243,27 @@ void run_decode(pa_decode_kind_t kind, at::Tensor& out, const at::Tensor& q,
   check_status(pa_validate_decode(kind, S, H, D, Hkv, NB, (int32_t)block_size, (int32_t)x, MB));
   if (S == 0) return;
 
-  // Split-K with equal lengths, known from the check above: the single-launch
-  // plan (host grid, splits merged in the launch) has no empty work-groups to
-  // avoid and no schedule to build first.  Same box, alternating, schedule ->
-  // grid: config 2's shape 27.25 -> 24.79 us; Llama 32/8 8 x 32k FP16 165.2 ->
-  // 157.8 (INT8 91.8 -> 89.8), 64k 320.8 -> 315.6 (174.3 -> 171.5), 128k INT8
-  // 343.3 -> 341.0; only 128k FP16 (4 GiB) turns, 656.1 -> 672.7.
-  if (equal_lens && (kind == PA_DECODE_SPLITK_F16 || kind == PA_DECODE_SPLITK_I8) &&
-      (int64_t)S * Hkv * max_ctx * D * (int8 ? 2 : 4) <= (int64_t(2) << 30))
+  // Which plan serves the call, where the check above has seen the lengths.  The
+  // single-launch plan (host grid) makes no schedule first but sizes every
+  // sequence for the longest; the in-kernel schedule of the split-K kinds
+  // balances what is there.  Both merge their splits in the launch.  Near-equal
+  // lengths (a mean of at least 0.7 of the maximum) take the grid under the split-K names, up to
+  // 2 GiB of K/V (equal 128k fp16, 4 GiB, turns: 656 -> 673 us); a mean below 0.6 of the
+  // maximum takes the schedule under the single-launch names, above the 64 MiB from
+  // which split-K calls are scheduled at all.  MI355X, grid / schedule in us: lengths within
+  // 1.1x (mean 0.95 of the maximum) 16 x 4000 32/8 fp16 45.8 / 51.2, 50 x 3000 8/8 D 64 53.8 / 68.7;
+  // within 1.7x (0.79) 38.8 / 42.2 (40 x 4000 12/2), 49.7 / 53.5 (INT8 60 x 6000 12/2); within 2.5x (0.7)
+  // 77.0 / 74.9 and 48.9 / 49.4; lognormal (0.3-0.4) 98.5 / 71.7, 63.1 / 42.5, INT8 87.4 / 57.9, D 256
+  // 56.4 / 33.7, MQA INT8 59.1 / 39.6, 200 x 1000 32/8 INT8 131 / 118.
+  const bool splitk = kind == PA_DECODE_SPLITK_F16 || kind == PA_DECODE_SPLITK_I8;
+  const int64_t bound = (int64_t)S * Hkv * max_ctx * D * (int8 ? 2 : 4);
+  const bool large = bound > (int64_t(64) << 20);
+  if (splitk && mean_ctx > 0 && bound <= (int64_t(2) << 30) &&
+      (mean_ctx == max_ctx || (large && (int64_t)mean_ctx * 10 >= (int64_t)max_ctx * 7)))
     kind = int8 ? PA_DECODE_WARP_I8 : PA_DECODE_WARP_F16;
+  else if (!splitk && mean_ctx > 0 && large && (int64_t)mean_ctx * 10 < (int64_t)max_ctx * 6 &&
+           S <= kMaxScheduledSeqs && partition_tokens == 0)
+    kind = int8 ? PA_DECODE_SPLITK_I8 : PA_DECODE_SPLITK_F16;
 
   const at::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
   hipStream_t stream = at::hip::getCurrentHIPStreamMasqueradingAsCUDA(q.get_device()).stream();

@@ -93,9 +93,9 @@ pa_status_t pa_check_context_lens(const int32_t* host_context_lens, int32_t num_
                                   int32_t* max_len);
 
 /* Range of context lengths on the device, for that check without a copy and a
- * synchronization.  out[0] = tag << 32 | minimum and out[1] = tag << 32 | maximum, each
- * word stored once, at system scope: with `out` in coherent host memory the caller polls
- * both words for its tag.  num_seqs >= 1. */
+ * synchronization.  out[0], out[1] and out[2] = tag << 32 | the minimum, the maximum and
+ * the mean (towards zero), each word stored once, at system scope: with `out` in coherent
+ * host memory the caller polls the three words for its tag.  num_seqs >= 1. */
 pa_status_t pa_context_lens_range(const int32_t* context_lens, int32_t num_seqs, uint64_t* out,
                                   uint32_t tag, pa_stream_t stream);
 

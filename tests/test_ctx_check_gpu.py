@@ -1,7 +1,8 @@
 """GPU tests of the ops' context-length check (the reference's `min >= 1` rule,
 paged_attention_v3_warp.cu:147-148), whose result a kernel writes where the
 host polls: positions of the extremes, batches around the reduction's sizes,
-work queued before it, several streams and threads, and capture."""
+work queued before it, several streams and threads, and the plan that the
+lengths choose."""
 
 import threading
 
@@ -103,3 +104,43 @@ def test_non_contiguous_lengths_are_still_refused():
     wide = torch.stack([x[4], x[4]], dim=1)
     with pytest.raises(RuntimeError, match="contiguous"):
         call(x[:4] + (wide[:, 0],))
+
+
+# lengths whose mean lies below 0.6, above 0.7 and between, of a launch above the 64 MiB
+# (bound: every sequence at the longest) from which the lengths choose the plan
+@pytest.mark.parametrize("pattern", ["ragged", "near_equal", "between", "equal"])
+@pytest.mark.parametrize("variant", ["warp", "splitk", "warp_int8", "splitk_int8"])
+def test_every_plan_gives_the_same_attention(pattern, variant):
+    import pa_int8
+
+    S, H, HKV, D, bs, top = 20, 8, 4, 128, 16, 4100
+    lens = {"ragged": [top] + [40 + 97 * i for i in range(S - 1)],
+            "near_equal": [top - 13 * i for i in range(S)],
+            "between": [top if i % 3 else 1000 for i in range(S)],
+            "equal": [top] * S}[pattern]
+    g = torch.Generator(device=DEV).manual_seed(len(pattern))
+    nblk = -(-top // bs)
+    nb = S * nblk
+    bt = torch.randperm(nb, device=DEV, generator=g).to(torch.int32).view(S, nblk)
+    q = torch.randn(S, H, D, device=DEV, generator=g).half()
+    ctx = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    int8 = variant.endswith("int8")
+    if int8:
+        kc = torch.randint(-127, 128, (nb, HKV, D // 8, bs, 8), device=DEV, generator=g).to(torch.int8)
+        vc = torch.randint(-127, 128, (nb, HKV, D, bs), device=DEV, generator=g).to(torch.int8)
+        ks, vs = (0.01 + 0.02 * torch.rand(nb, HKV, bs, device=DEV, generator=g) for _ in range(2))
+        extra = (ks, vs)
+    else:
+        kc = torch.randn(nb, HKV, D // 8, bs, 8, device=DEV, generator=g).half()
+        vc = torch.randn(nb, HKV, D, bs, device=DEV, generator=g).half()
+        ks = vs = None
+        extra = ()
+    ops = pa_int8.VARIANTS_INT8 if int8 else pa_int8.VARIANTS
+    got = ops[variant](torch.empty_like(q), q, kc, vc, *extra, bt, ctx, 0.09, bs)
+    other = variant.replace("warp", "splitk") if "warp" in variant else variant.replace("splitk", "warp")
+    for name in (variant, other):
+        want = pa_int8.decode(name, torch.empty_like(q), q, kc, vc, bt, ctx, 0.09, bs, k_scales=ks,
+                              v_scales=vs, check=False)
+        # both round an fp32 result to fp16: two roundings apart, and the fp16 softmax
+        # weights of differently cut splits (2^-11 each, averaged over the tokens)
+        torch.testing.assert_close(got.float(), want.float(), rtol=4e-3, atol=1e-3)
