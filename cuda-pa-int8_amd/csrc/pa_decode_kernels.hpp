@@ -1670,9 +1670,13 @@ __device__ __forceinline__ uint32_t one_round_partition(const DecodeShape& sh, c
   auto up = [](uint32_t v) { return (v + kIterTokens - 1) / kIterTokens * kIterTokens; };
   const uint32_t lo = (uint32_t)sa.pmin_uniform, hi = (uint32_t)sa.pmax;
   if (uniform) {
+    // (reciprocals instead of integer divisions, each a long sequence at the start of
+    // every launch; the half and the last step make up for their rounding)
+    const float ru = __builtin_amdgcn_rcpf((float)units);
     for (int r = 1; r <= 4; ++r) {
-      const uint32_t n = (uint32_t)(cus * r) / units;
-      const uint32_t p = up((b + n - 1) / n);
+      const uint32_t n = (uint32_t)(((float)(cus * r) + 0.5f) * ru);
+      uint32_t p = up((uint32_t)((float)b * __builtin_amdgcn_rcpf((float)n)));
+      p = (uint64_t)p * n < b ? p + kIterTokens : p;
       if (p <= hi) return p < lo ? lo : p;
     }
     return 0;
