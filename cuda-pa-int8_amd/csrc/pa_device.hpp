@@ -103,8 +103,8 @@ __device__ __forceinline__ void i8x4_to_biased_h2(uint32_t w, uint32_t& lo, uint
   hi = __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u);
 }
 
-// A load of data that is read once (cache tiles, inputs of the write
-// kernels): the non-temporal hint keeps it from being retained in the caches.
+// A load of data that is read once (the decode kernels' cache tiles): the
+// non-temporal hint keeps it from being retained in the caches.
 // On MI355X it raised the decode kernels' streaming rate from about 5.9 to
 // 6.4 TB/s (FP16, config 3 and config 4 shapes).
 template <typename T>
