@@ -1526,7 +1526,6 @@ struct SchedArgs {
   int pmin, pmax;     // partition bounds (multiples of kIterTokens)
   int pmin_uniform;   // lower bound when all lengths are equal (one item per work-group)
   float fill_scale;   // 1024 * kv heads * head chunks / CUs (see the ragged floor below)
-  float one_round_min;   // tokens per CU from which one_round_partition takes ragged lengths
 };
 
 constexpr int kShortBuckets = 4;   // (their counts pack into one 64-bit word)
@@ -1639,6 +1638,36 @@ __device__ __forceinline__ uint32_t wave_scan_dpp(uint32_t v) {
   return v + (row > 0 ? r0 : 0u) + (row > 1 ? r1 : 0u) + (row > 2 ? r2 : 0u);
 }
 
+// The partition of equal lengths (at most 64 sequences of b tokens): the fewest rounds of
+// one item per CU, up to 4, that the partition's upper bound allows, or 0 where there is
+// none.  Two items on one CU take about twice as long as one while the rest of the chip is
+// idle, so the items must not outnumber the CUs by a few; the rule from the token total
+// below it counts whole thousands of tokens and did.  MI355X, one item per CU rounded up ->
+// this, us: 17 x 21128 at 12/2 heads 82.9 -> 63.9 (INT8 49.1 -> 37.4), 5 x 50000 32/8 190.5 ->
+// 158.8.
+// Ragged lengths keep about four items per work-group.  One round of items half again as
+// long as a CU's share ran 5-20% faster on them (24 x 900-9000 8/4 head_dim 256 fp16 113 -> 97
+// us), but every wave keeps the softmax weights of an item relative to one running maximum, and
+// the longer the item, the fewer of them are exact: the outputs' distance from 64 bits grew
+// by 1.2-2.6% (that shape 2.68e-4 -> 2.75e-4, ten seeds, each mean within 0.01e-4).
+__device__ __forceinline__ uint32_t equal_partition(const DecodeShape& sh, const SchedArgs& sa,
+                                                    int cus, uint32_t b) {
+  const uint32_t units = (uint32_t)(sh.num_seqs * sh.num_kv_heads * sh.nchunk);
+  if (units > (uint32_t)cus || sa.pmin >= sa.pmax) return 0;   // (forced partitions stay)
+  const uint32_t lo = (uint32_t)sa.pmin_uniform, hi = (uint32_t)sa.pmax;
+  // (reciprocals instead of integer divisions, each a long sequence at the start of
+  // every launch; the half and the last step make up for their rounding)
+  const float ru = __builtin_amdgcn_rcpf((float)units);
+  for (int r = 1; r <= 4; ++r) {
+    const uint32_t n = (uint32_t)(((float)(cus * r) + 0.5f) * ru);
+    uint32_t p = (uint32_t)((float)b * __builtin_amdgcn_rcpf((float)n));
+    p = (p + kIterTokens - 1) / kIterTokens * kIterTokens;
+    p = (uint64_t)p * n < b ? p + kIterTokens : p;
+    if (p <= hi) return p < lo ? lo : p;
+  }
+  return 0;
+}
+
 // The schedule of at most 64 sequences, one per lane: every wave derives it
 // on its own with wave-wide reductions and DPP scans, wave 0 writes the
 // tables, and one barrier publishes them; the same tables
@@ -1647,67 +1676,6 @@ __device__ __forceinline__ uint32_t wave_scan_dpp(uint32_t v) {
 // bench's shapes (same box, alternating): config 2 split-K 28.73 -> 27.55 us,
 // config 4 32k INT8 90.43 -> 89.15 (FP16 166.61 -> 165.45), 8 x 32k MQA 35.08
 // -> 34.05 (INT8 28.49 -> 27.15); 128k even.
-// The partition that lets a launch of at most 64 sequences finish in one round of
-// work-groups, one per CU (equal lengths: in the fewest rounds, up to 4), or 0 where
-// there is none worth taking.  Two items on one CU take about twice as long as one,
-// while the chip's bandwidth is shared by fewer: a few items more than CUs cost
-// far more than some CUs left idle, up to items half again as long as a CU's share
-// of the tokens.  Lane = sequence (c: its length); t, b: tokens / 1024 and the longest.
-// MI355X, about four items per work-group (or one per CU rounded up) -> this, us:
-// ragged 24 x 900-9000 at 8/4 heads, head_dim 256 fp16 117 -> 97.6 (INT8 64.6 -> 60.6); 16 x
-// 1000-8000 32/8 57.3 -> 51.1 (INT8 36.1 -> 31.2); 30 x median 4096 16/4 69.6 -> 66.0; 8 x 8000-24000
-// 32/8 89.8 -> 81.2; equal 17 x 21128 12/2 82.9 -> 63.9 (49.1 -> 37.4), 5 x 50000 32/8 190.5 ->
-// 158.8.  Ragged launches of less than kOneRoundMinBytes per CU keep the finer items (INT8 40 x
-// median 4096 8/1, 256 KB per CU: 20.0 against 21.0; fp16 20 x 2300-5700 16/4 head_dim 64, 313 KB:
-// 20.3 -> 19.5).
-constexpr int kOneRoundMinBytes = 288 << 10;
-__device__ __forceinline__ uint32_t one_round_partition(const DecodeShape& sh, const SchedArgs& sa,
-                                                        int cus, uint32_t c, bool in, uint32_t t,
-                                                        uint32_t b, bool uniform) {
-  const uint32_t h = (uint32_t)(sh.num_kv_heads * sh.nchunk);
-  const uint32_t units = (uint32_t)sh.num_seqs * h;
-  if (units > (uint32_t)cus || sa.pmin >= sa.pmax) return 0;   // (forced partitions stay)
-  auto up = [](uint32_t v) { return (v + kIterTokens - 1) / kIterTokens * kIterTokens; };
-  const uint32_t lo = (uint32_t)sa.pmin_uniform, hi = (uint32_t)sa.pmax;
-  if (uniform) {
-    // (reciprocals instead of integer divisions, each a long sequence at the start of
-    // every launch; the half and the last step make up for their rounding)
-    const float ru = __builtin_amdgcn_rcpf((float)units);
-    for (int r = 1; r <= 4; ++r) {
-      const uint32_t n = (uint32_t)(((float)(cus * r) + 0.5f) * ru);
-      uint32_t p = up((uint32_t)((float)b * __builtin_amdgcn_rcpf((float)n)));
-      p = (uint64_t)p * n < b ? p + kIterTokens : p;
-      if (p <= hi) return p < lo ? lo : p;
-    }
-    return 0;
-  }
-  // (float arithmetic: the row counts only steer the choice, and every
-  // work-group evaluates the same operations on the same values)
-  const float share = ((float)t + 0.5f * (float)sh.num_seqs) *
-                      (1024.f * (float)h * __builtin_amdgcn_rcpf((float)cus));
-  if (share < sa.one_round_min) return 0;
-  constexpr int kTries = 4;
-  constexpr float kFactor[kTries] = {1.1f, 1.2f, 1.35f, 1.5f};
-  uint32_t part[kTries], rows[kTries / 2];
-#pragma unroll
-  for (int k = 0; k < kTries; ++k) {
-    const uint32_t p = up((uint32_t)(share * kFactor[k]) + 1);
-    part[k] = p < lo ? lo : p;
-    const float q = __builtin_ceilf((float)c * __builtin_amdgcn_rcpf((float)part[k]));
-    const uint32_t n = in ? (uint32_t)fminf(fmaxf(q, 1.f), 1023.f) : 0u;
-    rows[k / 2] = (k & 1) ? rows[k / 2] | (n << 16) : n;   // 64 x 1023 rows fit 16 bits
-  }
-  uint32_t best = 0;
-#pragma unroll
-  for (int k = kTries / 2 - 1; k >= 0; --k) {
-    const uint32_t n2 =
-        (uint32_t)__builtin_amdgcn_readfirstlane((int)wave_reduce_u(rows[k], OpAddU()));
-    if ((n2 >> 16) * h <= (uint32_t)cus && part[2 * k + 1] <= hi) best = part[2 * k + 1];
-    if ((n2 & 0xFFFFu) * h <= (uint32_t)cus && part[2 * k] <= hi) best = part[2 * k];
-  }
-  return best;
-}
-
 template <int NTH>
 __device__ __forceinline__ Schedule build_schedule_small(const int* __restrict__ ctxl,
                                                          const DecodeShape& sh,
@@ -1743,9 +1711,11 @@ __device__ __forceinline__ Schedule build_schedule_small(const int* __restrict__
     f = (f + kIterTokens - 1) / kIterTokens * kIterTokens;
     const uint64_t lo = (sc.uniform || f < (uint64_t)sa.pmin_uniform) ? (uint64_t)sa.pmin_uniform : f;
     part = part < lo ? lo : (part > (uint64_t)sa.pmax ? (uint64_t)sa.pmax : part);
-    const uint32_t one = one_round_partition(
-        sh, sa, (int)((gridDim.x + kGroupsPerCU - 1) / kGroupsPerCU), (uint32_t)c, in, t, b, sc.uniform);
-    if (one != 0) part = one;
+    if (sc.uniform) {
+      const uint32_t eq =
+          equal_partition(sh, sa, (int)((gridDim.x + kGroupsPerCU - 1) / kGroupsPerCU), b);
+      if (eq != 0) part = eq;
+    }
     const uint64_t top = ((uint64_t)(b > 0 ? b : 1) + kIterTokens - 1) / kIterTokens * kIterTokens;
     sc.partition = (int)(part < top ? part : top);
   }
@@ -2430,8 +2400,7 @@ hipError_t launch_decode_tiles(const DecodeLaunch& l) {
     const int cus = (l.groups + kGroupsPerCU - 1) / kGroupsPerCU;
     const SchedArgs sa{l.queue, l.rows_max, l.pmin, l.pmax, l.pmin_uniform,
                        1024.f * (float)(l.shape.num_kv_heads * l.shape.nchunk) /
-                           (float)(cus > 0 ? cus : 1),
-                       (float)kOneRoundMinBytes / (float)(2 * D * (I8 ? 1 : 2))};
+                           (float)(cus > 0 ? cus : 1)};
     const auto* q = static_cast<const half_t*>(l.q);
     const auto* kc = static_cast<const uint8_t*>(l.k_cache);
     const auto* vc = static_cast<const uint8_t*>(l.v_cache);
