@@ -116,25 +116,42 @@ struct Plan {
   bool fused = false;     // splits merged in the same launch (last-arriving work-group)
 };
 
-// Tokens per split of `units` units of `ctx` tokens (row_bytes of K/V each): a
-// multiple of `step` in [lo, hi].  What a launch costs, in tokens of a CU's time:
-// the rounds its work-groups take, one per CU at a time, times a split; no less than
+// Tokens per split of `units` units of `ctx` tokens (row_bytes of K/V each): in [lo, hi].
+// The fixed target, `groups` work-groups in as few splits as possible, stands where its
+// work-groups fit one round of the CUs: there a split is bound by its own serial chunks and
+// more, shorter ones are what helps.  (Weighed by the cost below, whose constants are a busy
+// chip's bandwidth, such launches kept long splits: 4 x 2000 8/1 INT8 head_dim 64 one split
+// 10.1 us against four 6.9, 1 x 12000 8/1 INT8 head_dim 8 32.6 against 8.4, 64 x 1000 12/2
+// fp16 17.2 against 15.8; over 81 such shapes of head_dim 8-256 the cost's plans took 0.84 to
+// 3.9 times as long, 1.14 in the geometric mean.)
+//
+// Past one round, a launch is weighed by what it costs in tokens of a CU's time: the
+// rounds its work-groups take, one per CU at a time, times a split; no less than
 // the work spread over three quarters of the CUs, which already draw the full
 // bandwidth; a fixed cost per round (128 KB worth: block ids, first rows, epilogue)
-// and one for merging at all (200 KB).  Work-groups just past a whole round are the
+// and one for merging at all (200 KB), both in rows of at least 256 bytes (an iteration
+// of smaller rows takes no less time).  Work-groups just past a whole round are the
 // expensive case: the CUs that hold two of them take twice as long, while the rest
-// of the chip is idle.  Candidates: per number of rounds, the most splits that fit and
-// the fewest that fill three quarters.  MI355X, fixed 256-work-group target ->
+// of the chip is idle.  Candidates (multiples of `step` tokens): per number of rounds, the
+// most splits that fit and the fewest that fill three quarters.  MI355X, fixed target ->
 // this rule, us (fp16 / INT8, head_dim 128): 17 x 21128 at 12/2 heads (34 units) 84.4 ->
 // 60 / 50.9 -> 36; 48 x 8192 12/2 87.8 -> 64.2 / 54.2 -> 39.4; 9 x 8192 32/8 66.2 ->
 // 51.0 / 41.7 -> 30.8; 70 x 2048 12/2 38.6 -> 28.4 / 24.3 -> 16.9; 36 x 3000 32/8 (288
 // units, more than a round unsplit) 88.4 -> 80.1 / 53.5 -> 47.1; head_dim 256: 12 x 6000 8/4
-// 55.6 -> 48.0 / 35.3 -> 31.3; the same plans where the units divide the CUs.
+// 55.6 -> 48.0 / 35.3 -> 31.3; 486 shapes past one round 1.20 times as fast in the geometric
+// mean (a tenth above 1.40, three below 0.96).  Where the tables are filled to only 0.2-0.6 of the
+// planned length (835 launches), it is chance how the busy splits fall: 1.07 in the geometric
+// mean, a tenth below 0.88, a tenth above 1.43.
 long long pick_partition(long long ctx, long long units, long long lo, long long hi, long long step,
-                         long long row_bytes) {
+                         long long groups, long long row_bytes) {
   const long long cus = kTargetWaves / 8;
+  long long target = (ctx * units + groups - 1) / groups;
+  target = (target + kMinPartition - 1) / kMinPartition * kMinPartition;
+  target = std::min(std::max(target, lo), hi);
+  if (units * ((ctx + target - 1) / target) <= cus) return target;
   const long long fill = (ctx * units * 4 + 3 * cus - 1) / (3 * cus);
-  const long long round_cost = (128 << 10) / row_bytes, merge_cost = (200 << 10) / row_bytes;
+  const long long row = std::max<long long>(row_bytes, 256);
+  const long long round_cost = (128 << 10) / row, merge_cost = (200 << 10) / row;
   const long long n_min = (ctx + hi - 1) / hi, n_max = std::max(n_min, (ctx + lo - 1) / lo);
   long long best = 0, best_cost = 0;
   auto consider = [&](long long n) {
@@ -253,11 +270,10 @@ Plan make_plan(pa_decode_kind_t kind, int num_seqs, int num_heads, int num_kv_he
     part = std::min<long long>(partition_tokens, hi);
   } else {
     const int plan_waves = quad ? 8 : p.waves;   // the group size the shortest split assumes
-    const long long lo = head_dim > 128 ? kMinPartition / 2
-                                        : (long long)kMinPartition * plan_waves / 4;
+    const long long lo = (long long)kMinPartition * plan_waves / 4;
     part = pick_partition(ctx, std::max(1, p.units), lo, hi,
                           head_dim > 128 ? kMinPartition / 2 : kMinPartition,
-                          2ll * head_dim * (is_f16(kind) ? 2 : 1));
+                          kTargetWaves / plan_waves, 2ll * head_dim * (is_f16(kind) ? 2 : 1));
   }
   part = (part + pa::kIterTokens - 1) / pa::kIterTokens * pa::kIterTokens;
   part = std::min<long long>(part, (ctx + pa::kIterTokens - 1) / pa::kIterTokens * pa::kIterTokens);

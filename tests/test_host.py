@@ -184,6 +184,54 @@ def test_single_launch_group_sizes(lib):
     assert p["waves"] == 8, p
 
 
+@pytest.mark.parametrize("kind,head_bytes", [(0, 2), (2, 1)])
+def test_split_plan_of_one_round_is_the_fixed_target(lib, kind, head_bytes):
+    """Where the fixed target's work-groups (256 of 8 waves, 512 of 4 at head_dim > 128; splits of
+    at least 512 or 256 tokens) fit one round of the 256 CUs, they are the plan, whatever the
+    width of the rows; it always does so at head_dim <= 128 where the units divide the
+    CUs.  Beyond, a launch never ends up with more rounds than the target's."""
+    info = (ctypes.c_int32 * 7)()
+    fits = past = 0
+    for d in (8, 16, 32, 64, 80, 96, 128, 192, 256):
+        for h, hkv in ((8, 8), (8, 2), (8, 1), (16, 4), (12, 2), (32, 8), (32, 1)):
+            for s in (1, 2, 3, 4, 5, 7, 8, 9, 16, 17, 32, 64, 70, 128):
+                for ctx in (64, 512, 1000, 2000, 4096, 6000, 12000, 21128, 65536):
+                    assert lib.pa_decode_plan_detail(kind, s, h, d, hkv, 16, -(-ctx // 16), ctx, 0,
+                                                     info, 7) == 0
+                    part, splits, waves, tile = info[:4]
+                    units = s * hkv * (h // hkv // tile)
+                    groups, lo = (512, 256) if d > 128 else (256, 512)
+                    hi = (4096 if d > 128 else 8192) * waves // 4
+                    want = -(-(-(-ctx * units // groups)) // 256) * 256
+                    want = min(min(max(want, lo), hi), -(-ctx // 64) * 64)
+                    n = -(-ctx // want)
+                    if units * n <= 256:
+                        assert (part, splits) == (want, n), (d, h, hkv, s, ctx, part, want)
+                        fits += 1
+                    else:
+                        assert -(-units * splits // 256) <= max(-(-units * n // 256), 4), (d, s, ctx)
+                        past += 1
+                    if d <= 128 and 256 % units == 0 and ctx * units <= 256 * hi:
+                        assert units * n <= 256 and (part, splits) == (want, n)
+    assert fits > 2000 and past > 1000
+
+
+def test_split_plans_named_shapes(lib):
+    """Plans of shapes whose times are quoted beside the planner: few short rows keep the
+    splits that fill the chip, launches just past a round take whole ones."""
+    info = (ctypes.c_int32 * 7)()
+    for kind, s, h, hkv, d, ctx, splits in (
+            (2, 1, 8, 1, 8, 12000, 24), (2, 1, 8, 1, 16, 6000, 12), (2, 4, 8, 1, 64, 2000, 4),
+            (2, 1, 8, 8, 64, 2048, 4), (0, 1, 8, 1, 16, 3000, 6), (0, 64, 12, 2, 128, 1000, 2),
+            (2, 16, 32, 8, 64, 4096, 2), (2, 4, 8, 8, 128, 1000, 2), (0, 8, 8, 1, 256, 2000, 8),
+            # past one round (34, 96, 72, 140, 288 and, at head_dim 256, 48 units)
+            (0, 17, 12, 2, 128, 21128, 6), (0, 48, 12, 2, 128, 8192, 2), (0, 9, 32, 8, 128, 8192, 3),
+            (2, 70, 12, 2, 128, 2048, 1), (0, 36, 32, 8, 128, 3000, 2), (0, 12, 8, 4, 256, 6000, 5)):
+        assert lib.pa_decode_plan_detail(kind, s, h, d, hkv, 16, -(-ctx // 16), ctx, 0, info,
+                                         7) == 0
+        assert info[1] == splits, (kind, s, h, hkv, d, ctx, list(info))
+
+
 def test_small_split_k_launches_take_the_grid(lib):
     """Split-K launches that read at most 64 MB (bound: every sequence at the
     checked maximum, else at the table's capacity) take the single-launch
