@@ -63,6 +63,9 @@ constexpr int kKntMinPartition = 1024;          // non-temporal K rows from this
 // Split-K launches that read at most this much K/V (bound: every sequence at
 // the checked maximum or the block-table capacity) take the single-launch plan.
 constexpr long long kSplitKGridMaxBytes = 64ll << 20;
+// Split-K calls whose checked lengths are equal or nearly so take the single-launch
+// plan up to this much K/V.
+constexpr long long kCheckedGridMaxBytes = 2ll << 30;
 // Upper bound on resident decode work-groups used to size the partial
 // buffers of the in-kernel schedule (256 CUs x 2 groups on MI355X).
 constexpr int kSchedGroupsBound = 1024;
@@ -556,6 +559,41 @@ pa_status_t pa_check_context_lens(const int32_t* host_context_lens, int32_t num_
   }
   if (max_len) *max_len = mx;
   return PA_OK;
+}
+
+// Which plan serves a call whose lengths have been seen.  The single-launch plan (host
+// grid) makes no schedule first but sizes every sequence for the longest; the
+// in-kernel schedule of the split-K kinds balances what is there.  Both merge their
+// splits in the launch.  Near-equal lengths (a mean of at least 0.7 of the maximum) take the
+// grid under the split-K names, up to 2 GiB of K/V (equal 128k fp16, 4 GiB, turns: 656 -> 673
+// us); a mean below 0.6 of the maximum takes the schedule under the single-launch names, above
+// the size from which split-K calls are scheduled at all.  MI355X, grid / schedule in us:
+// lengths within
+// 1.1x (mean 0.95 of the maximum) 16 x 4000 32/8 fp16 45.8 / 51.2, 50 x 3000 8/8 D 64 53.8 / 68.7;
+// within 1.7x (0.79) 38.8 / 42.2 (40 x 4000 12/2), 49.7 / 53.5 (INT8 60 x 6000 12/2); within 2.5x (0.7)
+// 77.0 / 74.9 and 48.9 / 49.4; lognormal (0.3-0.4) 98.5 / 71.7, 63.1 / 42.5, INT8 87.4 / 57.9, D 256
+// 56.4 / 33.7, MQA INT8 59.1 / 39.6, 200 x 1000 32/8 INT8 131 / 118.
+pa_decode_kind_t pa_decode_checked_kind(pa_decode_kind_t kind, int32_t num_seqs, int32_t num_heads,
+                                        int32_t head_dim, int32_t num_kv_heads,
+                                        int32_t block_size, int32_t max_blocks_per_seq,
+                                        int32_t max_len, int32_t mean_len,
+                                        int32_t partition_tokens) {
+  (void)num_heads, (void)block_size, (void)max_blocks_per_seq;
+  if (mean_len <= 0) return kind;
+  const bool f16 = is_f16(kind);
+  const long long bytes =
+      (long long)num_seqs * num_kv_heads * max_len * head_dim * 2 * (f16 ? 2 : 1);
+  const pa_decode_kind_t grid = f16 ? PA_DECODE_WARP_F16 : PA_DECODE_WARP_I8;
+  const pa_decode_kind_t sched = f16 ? PA_DECODE_SPLITK_F16 : PA_DECODE_SPLITK_I8;
+  if (!is_fused(kind) && mean_len == max_len) return bytes <= kCheckedGridMaxBytes ? grid : kind;
+  // (a caller that forces the partition or the distribution means this kind's)
+  if (bytes <= kSplitKGridMaxBytes || partition_tokens > 0 || g_schedule_mode != 0) return kind;
+  if (!is_fused(kind))
+    return bytes <= kCheckedGridMaxBytes && (long long)mean_len * 10 >= (long long)max_len * 7
+               ? grid
+               : kind;
+  return num_seqs <= pa::kSchedMaxSeqs && (long long)mean_len * 10 < (long long)max_len * 6 ? sched
+                                                                                           : kind;
 }
 
 pa_status_t pa_context_lens_range(const int32_t* context_lens, int32_t num_seqs, uint64_t* out,

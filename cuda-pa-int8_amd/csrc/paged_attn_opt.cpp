@@ -19,7 +19,6 @@
 namespace {
 
 constexpr int64_t kRefTile = 128;
-constexpr int32_t kMaxScheduledSeqs = 1024;   // batches the in-kernel schedule takes
 
 // Device memory of a decode call (include/pa_mi355x.h):
 //
@@ -243,27 +242,9 @@ void run_decode(pa_decode_kind_t kind, at::Tensor& out, const at::Tensor& q,
   check_status(pa_validate_decode(kind, S, H, D, Hkv, NB, (int32_t)block_size, (int32_t)x, MB));
   if (S == 0) return;
 
-  // Which plan serves the call, where the check above has seen the lengths.  The
-  // single-launch plan (host grid) makes no schedule first but sizes every
-  // sequence for the longest; the in-kernel schedule of the split-K kinds
-  // balances what is there.  Both merge their splits in the launch.  Near-equal
-  // lengths (a mean of at least 0.7 of the maximum) take the grid under the split-K names, up to
-  // 2 GiB of K/V (equal 128k fp16, 4 GiB, turns: 656 -> 673 us); a mean below 0.6 of the
-  // maximum takes the schedule under the single-launch names, above the 64 MiB from
-  // which split-K calls are scheduled at all.  MI355X, grid / schedule in us: lengths within
-  // 1.1x (mean 0.95 of the maximum) 16 x 4000 32/8 fp16 45.8 / 51.2, 50 x 3000 8/8 D 64 53.8 / 68.7;
-  // within 1.7x (0.79) 38.8 / 42.2 (40 x 4000 12/2), 49.7 / 53.5 (INT8 60 x 6000 12/2); within 2.5x (0.7)
-  // 77.0 / 74.9 and 48.9 / 49.4; lognormal (0.3-0.4) 98.5 / 71.7, 63.1 / 42.5, INT8 87.4 / 57.9, D 256
-  // 56.4 / 33.7, MQA INT8 59.1 / 39.6, 200 x 1000 32/8 INT8 131 / 118.
-  const bool splitk = kind == PA_DECODE_SPLITK_F16 || kind == PA_DECODE_SPLITK_I8;
-  const int64_t bound = (int64_t)S * Hkv * max_ctx * D * (int8 ? 2 : 4);
-  const bool large = bound > (int64_t(64) << 20);
-  if (splitk && mean_ctx > 0 && bound <= (int64_t(2) << 30) &&
-      (mean_ctx == max_ctx || (large && (int64_t)mean_ctx * 10 >= (int64_t)max_ctx * 7)))
-    kind = int8 ? PA_DECODE_WARP_I8 : PA_DECODE_WARP_F16;
-  else if (!splitk && mean_ctx > 0 && large && (int64_t)mean_ctx * 10 < (int64_t)max_ctx * 6 &&
-           S <= kMaxScheduledSeqs && partition_tokens == 0)
-    kind = int8 ? PA_DECODE_SPLITK_I8 : PA_DECODE_SPLITK_F16;
+  // The plan that suits the lengths, where the check above has seen them.
+  kind = pa_decode_checked_kind(kind, S, H, D, Hkv, (int32_t)block_size, MB, max_ctx, mean_ctx,
+                                (int32_t)partition_tokens);
 
   const at::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
   hipStream_t stream = at::hip::getCurrentHIPStreamMasqueradingAsCUDA(q.get_device()).stream();

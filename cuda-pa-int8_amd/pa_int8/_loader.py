@@ -80,6 +80,7 @@ PROTOTYPES = {
     "pa_validate_decode": (ctypes.c_int, [ctypes.c_int, _i32, _i32, _i32, _i32, _i32, _i32, _i32,
                                           _i32]),
     "pa_check_context_lens": (ctypes.c_int, [_p, _i32, ctypes.POINTER(_i32)]),
+    "pa_decode_checked_kind": (ctypes.c_int, [ctypes.c_int] + [_i32] * 9),
     "pa_decode_plan": (ctypes.c_int, [ctypes.c_int, _i32, _i32, _i32, _i32, _i32, _i32, _i32,
                                       _i32, ctypes.POINTER(_i32), ctypes.POINTER(_i32)]),
     "pa_decode_workspace_bytes": (_sz, [ctypes.c_int, _i32, _i32, _i32, _i32, _i32, _i32, _i32,

@@ -99,6 +99,19 @@ pa_status_t pa_check_context_lens(const int32_t* host_context_lens, int32_t num_
 pa_status_t pa_context_lens_range(const int32_t* context_lens, int32_t num_seqs, uint64_t* out,
                                   uint32_t tag, pa_stream_t stream);
 
+/* The kind to launch a decode of `kind` as, once the longest length and the mean
+ * length (towards zero, at least 1; equal to the longest only where all lengths are
+ * equal; <= 0: not known) have been read back.  NEW API, host only: both kinds of a cache type compute
+ * the same function; near-equal lengths run faster on the single-launch kinds' grid, uneven
+ * ones on the split-K kinds' in-kernel schedule.  A forced partition, or a distribution
+ * forced by pa_decode_set_schedule, keeps `kind` (equal lengths apart, whose
+ * split-K calls of up to 2 GiB of K/V always take the single launch). */
+pa_decode_kind_t pa_decode_checked_kind(pa_decode_kind_t kind, int32_t num_seqs, int32_t num_heads,
+                                        int32_t head_dim, int32_t num_kv_heads,
+                                        int32_t block_size, int32_t max_blocks_per_seq,
+                                        int32_t max_len, int32_t mean_len,
+                                        int32_t partition_tokens);
+
 /* Split plan of the grid form: how many tokens each work-group covers (a
  * multiple of 64) and how many splits the longest sequence needs.  (Under the
  * in-kernel schedule the kernel picks the partition on the device from the

@@ -269,6 +269,60 @@ def test_small_split_k_launches_take_the_grid(lib):
             lib.pa_decode_set_schedule(0)
 
 
+WARP, SPLITK, WARP8, SPLITK8 = 0, 1, 2, 3
+
+
+def checked_kind(lib, kind, seqs, longest, mean, hkv=8, heads=32, d=128, blocks=None, part=0):
+    blocks = -(-longest // 16) if blocks is None else blocks
+    return lib.pa_decode_checked_kind(kind, seqs, heads, d, hkv, 16, blocks, longest, mean, part)
+
+
+@pytest.mark.parametrize("warp,splitk,tokens", [(WARP, SPLITK, 1), (WARP8, SPLITK8, 2)])
+def test_checked_kind_edges(lib, warp, splitk, tokens):
+    """The kind a checked call is launched as, on both sides of every edge: the mean against
+    the longest length, 64 MiB, 2 GiB, 1024 sequences.  (4096 bytes a token in fp16.)"""
+    n = 1000 * tokens                                   # 20 x 1000 tokens: 78 MiB
+    f = lambda kind, mean, seqs=20, top=n, **kw: checked_kind(lib, kind, seqs, top, mean, **kw)  # noqa: E731
+    assert f(splitk, n * 7 // 10) == warp and f(splitk, n * 7 // 10 - 1) == splitk
+    assert f(splitk, n - 1) == warp and f(splitk, n) == warp
+    assert f(warp, n * 6 // 10) == warp and f(warp, n * 6 // 10 - 1) == splitk
+    assert f(warp, n) == warp and f(warp, 1) == splitk
+    # a mean that is not known changes nothing
+    assert f(splitk, 0) == splitk and f(warp, 0) == warp
+    # 64 MiB: uneven and near-equal lengths keep their kind up to it, equal ones never mind
+    edge = 1024 * tokens
+    assert f(warp, edge // 4, 16, edge) == warp and f(warp, edge // 4, 16, edge + 1) == splitk
+    assert f(splitk, edge - 9, 16, edge) == splitk and f(splitk, edge - 9, 16, edge + 1) == warp
+    assert f(splitk, edge, 16, edge) == warp
+    # 2 GiB
+    edge = 32768 * tokens
+    assert f(splitk, edge, 16, edge) == warp and f(splitk, edge + 1, 16, edge + 1) == splitk
+    assert f(splitk, edge - 9, 16, edge) == warp and f(splitk, edge - 9, 16, edge + 1) == splitk
+    assert f(warp, 9000, 16, edge + 1) == splitk
+    # the schedule takes at most 1024 sequences
+    assert f(warp, 100, 1024, n) == splitk and f(warp, 100, 1025, n) == warp
+
+
+@pytest.mark.parametrize("warp,splitk", [(WARP, SPLITK), (WARP8, SPLITK8)])
+def test_checked_kind_leaves_forced_choices_alone(lib, warp, splitk):
+    """A forced partition or distribution keeps the kind that the caller named (the grid's
+    reduce launch, the stream partition and the schedule are reached by it); equal lengths
+    under a split-K name take the single launch all the same."""
+    def all_cases(part):
+        return [checked_kind(lib, k, 20, 4000, mean, part=part)
+                for k in (warp, splitk) for mean in (1000, 2600, 3999, 4000)]
+
+    kept = [warp] * 4 + [splitk] * 3 + [warp]
+    assert all_cases(0) == [splitk, warp, warp, warp, splitk, splitk, warp, warp]
+    assert all_cases(512) == kept
+    for mode in (1, 2, 3):
+        assert lib.pa_decode_set_schedule(mode) == 0
+        try:
+            assert all_cases(0) == kept and all_cases(512) == kept
+        finally:
+            lib.pa_decode_set_schedule(0)
+
+
 def test_waves_override_hook(lib):
     assert lib.pa_decode_set_waves_per_group(3) == 2
     for w in (4, 8, 0):
