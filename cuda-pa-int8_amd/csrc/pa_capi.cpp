@@ -66,6 +66,10 @@ constexpr long long kSplitKGridMaxBytes = 64ll << 20;
 // Split-K calls whose checked lengths are equal or nearly so take the single-launch
 // plan up to this much K/V.
 constexpr long long kCheckedGridMaxBytes = 2ll << 30;
+// Scratch that a single-launch call may allocate for the schedule's partials in place of the
+// grid's (1024 sequences of up to 4000 tokens at 32 heads with tables of 128k tokens would
+// take 153 MB in fp16 and 289 MB in INT8; the grid takes 17 MB).
+constexpr size_t kCheckedSchedMaxScratch = 64u << 20;
 // Upper bound on resident decode work-groups used to size the partial
 // buffers of the in-kernel schedule (256 CUs x 2 groups on MI355X).
 constexpr int kSchedGroupsBound = 1024;
@@ -578,7 +582,6 @@ pa_decode_kind_t pa_decode_checked_kind(pa_decode_kind_t kind, int32_t num_seqs,
                                         int32_t block_size, int32_t max_blocks_per_seq,
                                         int32_t max_len, int32_t mean_len,
                                         int32_t partition_tokens) {
-  (void)num_heads, (void)block_size, (void)max_blocks_per_seq;
   if (mean_len <= 0) return kind;
   const bool f16 = is_f16(kind);
   const long long bytes =
@@ -592,8 +595,15 @@ pa_decode_kind_t pa_decode_checked_kind(pa_decode_kind_t kind, int32_t num_seqs,
     return bytes <= kCheckedGridMaxBytes && (long long)mean_len * 10 >= (long long)max_len * 7
                ? grid
                : kind;
-  return num_seqs <= pa::kSchedMaxSeqs && (long long)mean_len * 10 < (long long)max_len * 6 ? sched
-                                                                                           : kind;
+  if (num_seqs > pa::kSchedMaxSeqs || (long long)mean_len * 10 >= (long long)max_len * 6) return kind;
+  // The schedule's partials are sized for what the tables can hold (the kernel clamps
+  // lengths to them), the grid's for the longest length.
+  auto scratch = [&](pa_decode_kind_t k) {
+    return pa_decode_workspace_bytes(k, num_seqs, num_heads, head_dim, num_kv_heads, block_size,
+                                     max_blocks_per_seq, max_len, 0);
+  };
+  const size_t need = scratch(sched);
+  return need <= kCheckedSchedMaxScratch || need <= scratch(kind) ? sched : kind;
 }
 
 pa_status_t pa_context_lens_range(const int32_t* context_lens, int32_t num_seqs, uint64_t* out,

@@ -103,7 +103,8 @@ pa_status_t pa_context_lens_range(const int32_t* context_lens, int32_t num_seqs,
  * length (towards zero, at least 1; equal to the longest only where all lengths are
  * equal; <= 0: not known) have been read back.  NEW API, host only: both kinds of a cache type compute
  * the same function; near-equal lengths run faster on the single-launch kinds' grid, uneven
- * ones on the split-K kinds' in-kernel schedule.  A forced partition, or a distribution
+ * ones on the split-K kinds' in-kernel schedule (which a single-launch call takes only
+ * where its scratch is at most 64 MiB or no more than the grid's).  A forced partition, or a distribution
  * forced by pa_decode_set_schedule, keeps `kind` (equal lengths apart, whose
  * split-K calls of up to 2 GiB of K/V always take the single launch). */
 pa_decode_kind_t pa_decode_checked_kind(pa_decode_kind_t kind, int32_t num_seqs, int32_t num_heads,

@@ -323,6 +323,31 @@ def test_checked_kind_leaves_forced_choices_alone(lib, warp, splitk):
             lib.pa_decode_set_schedule(0)
 
 
+@pytest.mark.parametrize("warp,splitk", [(WARP, SPLITK), (WARP8, SPLITK8)])
+def test_checked_kind_bounds_the_scratch(lib, warp, splitk):
+    """A single-launch call takes the schedule only where its partials, sized for what the
+    tables can hold, stay within 64 MiB or within the grid's own."""
+    def scratch(kind, seqs, h, d, hkv, blocks, longest):
+        return lib.pa_decode_workspace_bytes(kind, seqs, h, d, hkv, 16, blocks, longest, 0)
+
+    assert scratch(splitk, 1024, 32, 128, 8, 8192, 4000) > 140 << 20
+    assert checked_kind(lib, warp, 1024, 4000, 1000, blocks=8192) == warp
+    assert checked_kind(lib, warp, 200, 4000, 1000, blocks=1024) == splitk
+    taken = 0
+    for seqs in (2, 20, 64, 256, 1024):
+        for longest in (1000, 8000, 60000):
+            for h, hkv in ((8, 8), (12, 2), (32, 8), (32, 1), (128, 8)):
+                for d in (64, 128, 256):
+                    for cap in (longest, 4 * longest, 1 << 17, 1 << 20):
+                        blocks = -(-cap // 16)
+                        args = (seqs, h, d, hkv, blocks, longest)
+                        if checked_kind(lib, warp, seqs, longest, longest // 3, hkv, h, d,
+                                        blocks) == splitk:
+                            taken += 1
+                            assert scratch(splitk, *args) <= max(64 << 20, scratch(warp, *args))
+    assert taken > 200
+
+
 def test_waves_override_hook(lib):
     assert lib.pa_decode_set_waves_per_group(3) == 2
     for w in (4, 8, 0):
