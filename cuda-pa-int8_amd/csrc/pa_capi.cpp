@@ -570,13 +570,12 @@ pa_status_t pa_check_context_lens(const int32_t* host_context_lens, int32_t num_
 // in-kernel schedule of the split-K kinds balances what is there.  Both merge their
 // splits in the launch.  Near-equal lengths (a mean of at least 0.7 of the maximum) take the
 // grid under the split-K names, up to 2 GiB of K/V (equal 128k fp16, 4 GiB, turns: 656 -> 673
-// us); a mean below 0.6 of the maximum takes the schedule under the single-launch names, above
-// the size from which split-K calls are scheduled at all.  MI355X, grid / schedule in us:
-// lengths within
-// 1.1x (mean 0.95 of the maximum) 16 x 4000 32/8 fp16 45.8 / 51.2, 50 x 3000 8/8 D 64 53.8 / 68.7;
-// within 1.7x (0.79) 38.8 / 42.2 (40 x 4000 12/2), 49.7 / 53.5 (INT8 60 x 6000 12/2); within 2.5x (0.7)
-// 77.0 / 74.9 and 48.9 / 49.4; lognormal (0.3-0.4) 98.5 / 71.7, 63.1 / 42.5, INT8 87.4 / 57.9, D 256
-// 56.4 / 33.7, MQA INT8 59.1 / 39.6, 200 x 1000 32/8 INT8 131 / 118.
+// us); a mean below half of the maximum takes the schedule under the single-launch names, above
+// the size from which split-K calls are scheduled at all.  MI355X, time of the grid over
+// the schedule's, geometric mean (first and last tenth), 420 batches of 2-500 sequences of uniform,
+// lognormal and two-level lengths, 64 MiB-3 GiB, by mean over maximum: below 0.4 1.20 (0.98, 1.51);
+// 0.4-0.5 1.13 (0.93, 1.37); 0.5-0.6 1.00 (0.89, 1.15); 0.6-0.7 1.00 (0.88, 1.16); 0.7-0.8 0.94
+// (0.84, 1.06); above 0.93 (0.80, 1.04).
 pa_decode_kind_t pa_decode_checked_kind(pa_decode_kind_t kind, int32_t num_seqs, int32_t num_heads,
                                         int32_t head_dim, int32_t num_kv_heads,
                                         int32_t block_size, int32_t max_blocks_per_seq,
@@ -595,7 +594,7 @@ pa_decode_kind_t pa_decode_checked_kind(pa_decode_kind_t kind, int32_t num_seqs,
     return bytes <= kCheckedGridMaxBytes && (long long)mean_len * 10 >= (long long)max_len * 7
                ? grid
                : kind;
-  if (num_seqs > pa::kSchedMaxSeqs || (long long)mean_len * 10 >= (long long)max_len * 6) return kind;
+  if (num_seqs > pa::kSchedMaxSeqs || (long long)mean_len * 2 >= max_len) return kind;
   // The schedule's partials are sized for what the tables can hold (the kernel clamps
   // lengths to them), the grid's for the longest length.
   auto scratch = [&](pa_decode_kind_t k) {

@@ -285,7 +285,7 @@ def test_checked_kind_edges(lib, warp, splitk, tokens):
     f = lambda kind, mean, seqs=20, top=n, **kw: checked_kind(lib, kind, seqs, top, mean, **kw)  # noqa: E731
     assert f(splitk, n * 7 // 10) == warp and f(splitk, n * 7 // 10 - 1) == splitk
     assert f(splitk, n - 1) == warp and f(splitk, n) == warp
-    assert f(warp, n * 6 // 10) == warp and f(warp, n * 6 // 10 - 1) == splitk
+    assert f(warp, n // 2) == warp and f(warp, n // 2 - 1) == splitk
     assert f(warp, n) == warp and f(warp, 1) == splitk
     # a mean that is not known changes nothing
     assert f(splitk, 0) == splitk and f(warp, 0) == warp
