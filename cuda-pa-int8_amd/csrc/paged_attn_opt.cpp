@@ -72,38 +72,47 @@ at::Tensor counters_for(const at::Tensor& like, hipStream_t stream, size_t bytes
 
 void check_status(pa_status_t st) { TORCH_CHECK(st == PA_OK, pa_status_string(st)); }
 
-// Result slots of the context-length check: coherent host memory that a kernel
-// writes and the host polls.  One 4 KB block for the process, kept until it ends
-// (the driver may still be mapping it when a thread ends); a call holds one slot
-// until its kernel has written it, and finding none free is no error.
-struct RangeSlots {
-  static constexpr int kSlots = 32;
-  uint64_t* mem = nullptr;                  // kSlots x 8 words (a line each)
-  std::atomic<uint32_t> taken{0};
-  std::atomic<uint32_t> tag{0};
-  RangeSlots() {
-    void* p = nullptr;
-    if (hipHostMalloc(&p, 4096, hipHostMallocCoherent | hipHostMallocMapped |
-                                    hipHostMallocPortable) == hipSuccess)
-      mem = static_cast<uint64_t*>(p);
-    else
-      (void)hipGetLastError();
-  }
-  int take() {
-    uint32_t t = taken.load();
-    while (mem != nullptr && t != 0xFFFFFFFFu) {
-      const int i = __builtin_ctz(~t);
-      if (taken.compare_exchange_weak(t, t | (1u << i))) return i;
+// Where the context-length check's kernel leaves its result: three words of coherent host
+// memory that the host polls, held by one call at a time (the ops hold the interpreter's
+// lock throughout, so no other call waits for it).  Kept until the process ends; asked for
+// again by the next call where the allocation was refused.
+struct LengthSlot {
+  std::mutex mu;              // guards everything below
+  uint64_t* mem = nullptr;
+  uint32_t tag = 0;
+  bool lost = false;          // a kernel whose end is unknown may still write it
+  int refuse = 0;             // test hook: this many requests go without
+  int64_t polled = 0;         // checks answered through it
+
+  uint64_t* get() {
+    if (refuse > 0) {
+      --refuse;
+      return nullptr;
     }
-    return -1;
+    if (mem == nullptr) {
+      // (allowed while another thread captures a stream)
+      hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+      const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+      void* p = nullptr;
+      if (hipHostMalloc(&p, 4096, hipHostMallocCoherent | hipHostMallocMapped |
+                                      hipHostMallocPortable) == hipSuccess)
+        mem = static_cast<uint64_t*>(p);
+      else
+        (void)hipGetLastError();
+      if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+    return lost ? nullptr : mem;
   }
-  void give(int i) { taken.fetch_and(~(1u << i)); }
 };
+LengthSlot& length_slot() {
+  static LengthSlot* s = new LengthSlot();
+  return *s;
+}
 
 // Smallest, largest and mean context length through a kernel that writes them where the
 // host polls.  False (nothing done) where that does not apply: lengths elsewhere
 // than on q's device or not dense (a later check reports them), a stream under
-// capture, no free slot.
+// capture, no host memory.
 bool polled_range(const at::Tensor& ctx, const at::Tensor& q, int32_t* mn, int32_t* mx,
                   int32_t* mean) {
   if (!ctx.is_cuda() || ctx.get_device() != q.get_device() || !ctx.is_contiguous() ||
@@ -112,20 +121,16 @@ bool polled_range(const at::Tensor& ctx, const at::Tensor& q, int32_t* mn, int32
   const at::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
   hipStream_t stream = at::hip::getCurrentHIPStreamMasqueradingAsCUDA(q.get_device()).stream();
   if (stream_capturing(stream)) return false;
-  static RangeSlots* slots = new RangeSlots();
-  const int i = slots->take();
-  if (i < 0) return false;
-  volatile uint64_t* w = slots->mem + 8 * i;
-  const uint32_t tag = slots->tag.fetch_add(1) + 1;
+  LengthSlot& slot = length_slot();
+  std::lock_guard<std::mutex> lk(slot.mu);
+  uint64_t* const mem = slot.get();
+  if (mem == nullptr) return false;
+  volatile uint64_t* w = mem;
+  const uint32_t tag = ++slot.tag;
   w[0] = w[1] = w[2] = (uint64_t)(tag - 1) << 32;   // whatever the slot holds is not this call's tag
   std::atomic_thread_fence(std::memory_order_seq_cst);
-  const pa_status_t st =
-      pa_context_lens_range(ctx.data_ptr<int32_t>(), (int32_t)ctx.numel(), slots->mem + 8 * i, tag,
-                            reinterpret_cast<pa_stream_t>(stream));
-  if (st != PA_OK) {
-    slots->give(i);
-    check_status(st);
-  }
+  check_status(pa_context_lens_range(ctx.data_ptr<int32_t>(), (int32_t)ctx.numel(), mem, tag,
+                                     reinterpret_cast<pa_stream_t>(stream)));
   // The stream may have other work before the kernel: poll for about as long as
   // a blocked wait costs more than it saves, then wait on the stream.
   const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(1);
@@ -137,7 +142,7 @@ bool polled_range(const at::Tensor& ctx, const at::Tensor& q, int32_t* mn, int32
     __builtin_ia32_pause();
     if ((spin & 63) == 63 && std::chrono::steady_clock::now() > until) {
       const hipError_t e = hipStreamSynchronize(stream);
-      // (after a failed wait the kernel's fate is unknown: its slot stays taken)
+      slot.lost = e != hipSuccess || !done();   // (the kernel's fate is unknown)
       TORCH_CHECK(e == hipSuccess, "context_lens check: ", hipGetErrorString(e));
       TORCH_CHECK(done(), "context_lens check: the kernel's result did not arrive");
     }
@@ -145,10 +150,9 @@ bool polled_range(const at::Tensor& ctx, const at::Tensor& q, int32_t* mn, int32
   *mn = (int32_t)(uint32_t)w[0];
   *mx = (int32_t)(uint32_t)w[1];
   *mean = (int32_t)(uint32_t)w[2];
-  slots->give(i);
+  ++slot.polled;
   return true;
 }
-
 
 // Which reference launcher's block_size rule an op repeats: the naive stage
 // checks none (paged_attention_naive.cu:135-140), the vectorised stage only a
@@ -546,6 +550,13 @@ PYBIND11_MODULE(paged_attn_opt, m) {
   m.def("cache_prefill", &cache_prefill,
         "one prompt's cache write with the rest of its last block zeroed; per-tensor scales "
         "taken from the rows when asked for (new op)");
+  m.def("_length_slot", [](int refuse) {
+    LengthSlot& s = length_slot();
+    std::lock_guard<std::mutex> lk(s.mu);
+    s.refuse = refuse;
+    return s.polled;
+  }, "test hook: the next `refuse` length checks find no host memory to poll; returns how many "
+     "checks have been answered by polling");
   m.def("version", []() { return std::string(pa_version()); });
 }
 

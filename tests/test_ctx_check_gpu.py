@@ -1,8 +1,9 @@
 """GPU tests of the ops' context-length check (the reference's `min >= 1` rule,
 paged_attention_v3_warp.cu:147-148), whose result a kernel writes where the
 host polls: positions of the extremes, batches around the reduction's sizes,
-work queued before it, several streams and threads, and the plan that the
-lengths choose."""
+work queued before it, calls from several threads and streams in turn (the ops hold the
+interpreter's lock, so one call's check ends before the next begins), and the plan that
+the lengths choose."""
 
 import threading
 
@@ -97,6 +98,29 @@ def test_threads_and_streams():
     for t in threads:
         t.join()
     assert not errors, errors[0]
+
+
+def test_without_host_memory_to_poll():
+    """A check that finds no memory to poll reads the lengths back by copy, with the same
+    refusals, and the next check polls again."""
+    import pa_int8
+
+    x = inputs(8)
+    want = unchecked(x)
+    slot = pa_int8.ext()._length_slot
+    n = slot(0)
+    for polled in (1, 0, 1):
+        slot(1 - polled)
+        assert torch.equal(call(x), want)
+        assert slot(0) == n + polled
+        n += polled
+    bad = x[:4] + (x[4].clone(),)
+    bad[4][7] = 0
+    out = torch.full_like(x[0], 7)
+    slot(1)
+    with pytest.raises(RuntimeError, match="context_lens must be >= 1"):
+        pa_int8.VARIANTS["warp"](out, *bad, 0.3, 16)
+    assert (out == 7).all() and slot(0) == n
 
 
 def test_non_contiguous_lengths_are_still_refused():
