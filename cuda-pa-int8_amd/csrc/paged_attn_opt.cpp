@@ -189,15 +189,15 @@ void run_decode(pa_decode_kind_t kind, at::Tensor& out, const at::Tensor& q,
     // One read-back for both the reference's `min >= 1` rule (v3:147-148) and the
     // split count (v4:213-214).
     int32_t mn = 0;
-    if (polled_range(context_lens, q, &mn, &max_ctx, &mean_ctx)) {
-      if (mn != max_ctx && mean_ctx == max_ctx) mean_ctx = max_ctx - 1;   // (equal means equal)
-    } else {
+    if (!polled_range(context_lens, q, &mn, &max_ctx, &mean_ctx)) {
       const auto mnmx = at::aminmax(context_lens);
-      const at::Tensor mm = at::stack({std::get<0>(mnmx), std::get<1>(mnmx)}).cpu();
-      mn = mm[0].item<int32_t>();
-      max_ctx = mm[1].item<int32_t>();
-      if (mn == max_ctx) mean_ctx = mn;
+      const at::Tensor r = at::stack({std::get<0>(mnmx).to(at::kLong), std::get<1>(mnmx).to(at::kLong),
+                                      context_lens.sum()}).cpu();
+      mn = (int32_t)r[0].item<int64_t>();
+      max_ctx = (int32_t)r[1].item<int64_t>();
+      mean_ctx = (int32_t)(r[2].item<int64_t>() / context_lens.numel());
     }
+    if (mn != max_ctx && mean_ctx == max_ctx) mean_ctx = max_ctx - 1;   // (equal means equal)
     TORCH_CHECK(mn >= 1, "context_lens must be >= 1 (empty sequences unsupported)");
   }
   if (int8) {

@@ -123,6 +123,41 @@ def test_without_host_memory_to_poll():
     assert (out == 7).all() and slot(0) == n
 
 
+def test_read_back_by_copy_chooses_the_same_plan():
+    """A check that finds no memory to poll takes the plan that the polled one takes (launches
+    above 64 MiB, whose splits show in the last bits)."""
+    import pa_int8
+
+    S, H, HKV, D, bs, top = 20, 8, 4, 128, 16, 4100
+    lens = [top] + [40 + 97 * i for i in range(S - 1)]
+    g = torch.Generator(device=DEV).manual_seed(3)
+    nblk = -(-top // bs)
+    kc = torch.randn(S * nblk, HKV, D // 8, bs, 8, device=DEV, generator=g).half()
+    vc = torch.randn(S * nblk, HKV, D, bs, device=DEV, generator=g).half()
+    bt = torch.arange(S * nblk, dtype=torch.int32, device=DEV).view(S, nblk)
+    q = torch.randn(S, H, D, device=DEV, generator=g).half()
+    slot = pa_int8.ext()._length_slot
+
+    def both(ctx, variant):
+        n = slot(0)
+        polled = call((q, kc, vc, bt, ctx), variant)
+        assert slot(1) == n + 1
+        copied = call((q, kc, vc, bt, ctx), variant)
+        assert slot(0) == n + 1                      # that one did not poll
+        again = call((q, kc, vc, bt, ctx), variant)
+        assert slot(0) == n + 2
+        assert torch.equal(polled, copied) and torch.equal(polled, again)
+        return polled
+
+    ragged = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    near = torch.tensor([top - 13 * i for i in range(S)], dtype=torch.int32, device=DEV)
+    # (the plans' own outputs differ, so the comparisons above can tell them apart)
+    assert not torch.equal(both(ragged, "warp"), unchecked((q, kc, vc, bt, ragged), "warp"))
+    assert not torch.equal(both(near, "splitk"), unchecked((q, kc, vc, bt, near), "splitk"))
+    both(torch.full_like(near, top), "splitk")
+    slot(0)
+
+
 def test_non_contiguous_lengths_are_still_refused():
     x = inputs(4)
     wide = torch.stack([x[4], x[4]], dim=1)
