@@ -26,7 +26,7 @@
 // continue sequences at any position, is written in whole cells whatever the
 // position of its tokens in the input.  The window's *loose* tokens, which
 // belong to no run (the ends of a sequence, decode appends, scattered slots), are
-// stored one by one.
+// stored one by one.  (The form for few rows takes a window as it is.)
 //
 // What bounds it: HBM, mixed reads and writes; small launches, latency.  Many
 // rows: one wave per (window, head), K then V, both loads out together; the
@@ -48,8 +48,7 @@
 // lanes that share a dim group with the 8 dims of that group; a store
 // instruction of a run therefore covers whole 128-byte lines of V at block size
 // 16, as it does of K, and no LDS is used.  Tokens outside runs are stored
-// element by element from the same registers (8 lines per instruction
-// instead of the 64 of a token-per-lane store).
+// element by element (write_loose).
 //
 // Quantizing multiplies by the reciprocal of the scale; an element whose
 // product lies too close to a rounding tie (or is not finite) is redone with
@@ -497,11 +496,16 @@ __device__ __forceinline__ void write_run(const WriteArgs& a,
 }
 
 // Writes one row of the window's loose tokens (t0 + k for the bits k of `loose`),
-// each at its own slot; sl: the slot of token t0 + i.
+// each at its own slot; sl: the slot of token t0 + i.  V goes out element by element: from the
+// transposed registers, 8 dims of a token per store instruction and 8 lanes, or, where most of the
+// tokens are neighbours in the cache (`together`), as loaded, 16 tokens of a dim (MI355X, INT8,
+// 8 chunks of 256 x 8 heads at slot 8: 7.1 / 6.8 us at block size 16, 10.9 / 6.8 at 64, fp16 9.4 / 7.1
+// and 12.9 / 6.6; 256 appends fp16 5.0 / 7.2).
 template <int D, WriteMode MODE, bool BF, bool PROBE>
 __device__ __forceinline__ void write_loose(const WriteArgs& a,
                                             const WriteLane<MODE != WriteMode::kF16>& ln, bool v,
-                                            int h, int t0, uint32_t loose, int64_t sl, const WriteRow<D>& r) {
+                                            int h, int t0, uint32_t loose, int64_t sl,
+                                            const WriteRow<D>& r, bool together) {
   constexpr bool I8 = MODE != WriteMode::kF16;
   constexpr int ESZ = I8 ? 1 : 2;
   constexpr int DG = WriteRow<D>::DG, JQ = WriteRow<D>::JQ;
@@ -525,6 +529,23 @@ __device__ __forceinline__ void write_loose(const WriteArgs& a,
       for (int j = 0; j < JQ; ++j)
         if (ln.qq + 4 * j < DG)
           *reinterpret_cast<Group*>(dst + (size_t)((ln.qq + 4 * j) * bs * 8 * ESZ)) = g[j];
+    }
+  } else if (together) {
+    if (mine) {
+      uint8_t* const dst =
+          static_cast<uint8_t*>(a.vc) + ((bh * D + 8 * ln.qq) * bs + off) * (int64_t)ESZ;
+#pragma unroll
+      for (int j = 0; j < JQ; ++j) {
+        if (ln.qq + 4 * j >= DG) continue;
+        uint32_t d[sizeof(Group) / 4];
+        __builtin_memcpy(d, &g[j], sizeof(Group));
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          uint8_t* const e = dst + (size_t)((32 * j + k) * bs * ESZ);
+          if constexpr (I8) *e = (uint8_t)(d[k / 4] >> (8 * (k & 3)));
+          else *reinterpret_cast<uint16_t*>(e) = (uint16_t)(d[k / 2] >> (16 * (k & 1)));
+        }
+      }
     }
   } else {
     const int64_t col = bh * D * bs + off;   // the token's column of its V tile
@@ -594,45 +615,63 @@ __global__ void __launch_bounds__(kWriteWaves * kWave) paged_write_kernel(WriteA
     for (int part = 0; part < 2; ++part) {
       WriteRow<D> r;
       load_row<D>(a, part != 0, h, t0, ln.i, ln.qq, r);
-      write_loose<D, MODE, BF, PROBE>(a, ln, part != 0, h, t0, win.loose, sl, r);
+      write_loose<D, MODE, BF, PROBE>(a, ln, part != 0, h, t0, win.loose, sl, r, false);
     }
   }
 }
 
-// The form for few rows (decode appends, short prompts), which are bound by
-// latency: one wave for each window, head, K or V, and run or loose tokens.  The
-// row is loaded together with the slots, at the window's own tokens (which it is
-// for loose tokens and for a run that starts the window).
+// The form for few rows (decode appends, short prompts and chunks), which are bound by
+// latency: one wave for each window, head, K or V.  The row is loaded together with the
+// slots, at the window's own tokens, and nothing waits for a second load: a window whose 16
+// tokens fill one cell is written as a run, all others token by token.  (Searching runs as the
+// form for many rows does, a run that starts inside its window had its row loaded again once
+// the slots were known, beside idle waves for the kind of token a window has none of.)
+// MI355X, with that search -> this, us: INT8 23 chunks of 32-42 tokens x 8 heads at odd
+// positions 5.9 -> 4.8, one of 601 5.6 -> 4.4 (blocks of 64 5.6 -> 4.2); 3 prompts of 1500-2000 x 1
+// head 6.1 -> 4.65; fp16 23 chunks, blocks of 64, 6.2 -> 3.8; 8 chunks of 192-256 x 8 heads INT8
+// 8.2 -> 6.8, fp16 6.6 -> 7.1 (7.25 before the search).
 template <int D, WriteMode MODE, bool BF, bool PROBE = false>
 __global__ void __launch_bounds__(kWriteWaves * kWave) paged_write_small_kernel(WriteArgs a) {
   const int item = blockIdx.x * (blockDim.x >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int win_no = item / (4 * a.hkv), sub = item - win_no * 4 * a.hkv;
-  const int t0 = win_no * 16, h = sub >> 2;
-  const bool v = sub & 1, loose = sub & 2;
+  const int win_no = item / (2 * a.hkv), sub = item - win_no * 2 * a.hkv;
+  const int t0 = win_no * 16, h = sub >> 1;
+  const bool v = sub & 1;
   if (t0 >= a.num_tokens) return;
   const WriteLane<MODE != WriteMode::kF16> ln;
-  WindowSlots ws;
-  ws.load(a, t0, ln.lane);
-  const int64_t sl = a.slots[min(t0 + ln.i, a.num_tokens - 1)];
+  const int tok = t0 + ln.i;
+  const bool in = tok < a.num_tokens;
+  int64_t sl = a.slots[in ? tok : a.num_tokens - 1];
   WriteRow<D> r;
   load_row<D>(a, v, h, t0, ln.i, ln.qq, r);
-  const Window win = find_runs(a, t0, ln.lane, ws);
-  if (loose) {
-    if (win.loose != 0) write_loose<D, MODE, BF, PROBE>(a, ln, v, h, t0, win.loose, sl, r);
-  } else if (win.run) {
-    if (win.start != 0) load_row<D>(a, v, h, t0 + win.start, ln.i, ln.qq, r);
-    write_run<D, MODE, BF, PROBE>(a, ln, v, h, t0 + win.start, win.slot, r);
+  const bool ok = in && sl >= 0 && sl < a.pool;
+  const int64_t slot = readlane64(sl, 0);   // token t0's (lane 0 holds it)
+  const bool run = a.bs >= 16 && (slot & 15) == 0 &&
+                   __builtin_amdgcn_ballot_w64(!ok || sl != slot + ln.i) == 0;
+  if (run) {
+    write_run<D, MODE, BF, PROBE>(a, ln, v, h, t0, slot, r);
+  } else {
+    // bit k: token t0 + k, which lane lane_token(k) of every 16 holds
+    const uint32_t held = (uint32_t)__builtin_amdgcn_ballot_w64(ok) & 0xFFFFu;
+    const uint32_t loose = (held & 0xF00Fu) | ((held & 0x0F00u) >> 4) | ((held & 0x00F0u) << 4);
+    // neighbours of the window's first or last token in the cache
+    const int64_t last = readlane64(sl, 15);
+    const bool near = ok && (sl == slot + ln.i || sl == last - (15 - ln.i));
+    const bool together = __popcll(__builtin_amdgcn_ballot_w64(near)) >= 32;
+    if (loose != 0) write_loose<D, MODE, BF, PROBE>(a, ln, v, h, t0, loose, sl, r, together);
   }
 }
 
-// Where the small form ends (its waves: four per window and head) and up to where
-// it runs in one-wave work-groups.  MI355X, head_dim 128, small / large form in us:
-// 3 prompts of 100-200 tokens x 8 heads (about 900 waves) INT8 4.8 / 8.7, fp16 3.4 /
-// 6.3; 12 of them (3400) 7.5 / 9.4, 6.0 / 7.2; one of 2000-4000 (4000 or more) 8.5 / 8.6, 7.2 /
-// 6.7.  Appends of 256 tokens x 8 heads run 6.4 us in one-wave work-groups and 5.7 us in
-// four-wave ones, of one token 3.38 and 3.45.
-constexpr int kSmallWaves = 4096;
-constexpr int kSmallSpreadWaves = 256;
+// Where the small form ends (its waves: two per window and head) and up to where it runs in
+// one-wave work-groups (which spread over more CUs).  MI355X, time of the small form over the
+// large one's, geometric mean of prompts and chunks x 8 heads, INT8 (bf16 rows and one given
+// scale alike) / fp16, by waves: 1700-2100 0.81 / 0.98, 2600-3100 0.77 / 0.94, 3100-3700 0.86 /
+// 1.01, 3700-4200 0.95 / 1.08 at head_dim 128; 2100-2600 0.83 / 0.97, 2600-3100 0.77 / 1.03, 3100-3700
+// 0.95 / 1.09, 3700-4200 1.08 / 1.26 at 256.  Work-groups of one wave against four: 300-370 waves
+// INT8 0.94, fp16 0.84; 512 0.97; 704 0.94, 0.92; 750-980 of one head 1.05, 1.10.
+template <int D, WriteMode MODE>
+constexpr int kSmallWaves = MODE == WriteMode::kF16 ? (D > 128 ? 2048 : 3072)
+                                                    : (D > 128 ? 3072 : 4096);
+constexpr int kSmallSpreadWaves = 704;
 
 template <int D, WriteMode MODE, bool BF, bool PROBE = false>
 hipError_t launch_write(const WriteLaunch& l) {
@@ -657,8 +696,8 @@ hipError_t launch_write(const WriteLaunch& l) {
   a.bs_log2 = __builtin_ctz((unsigned)l.block_size);
   a.pool = (int64_t)l.num_blocks * l.block_size;
   const long long windows = (a.num_tokens + 15ll) / 16;
-  const long long small = 4 * windows * l.num_kv_heads;
-  if (small <= kSmallWaves) {
+  const long long small = 2 * windows * l.num_kv_heads;
+  if (small <= kSmallWaves<D, MODE>) {
     const int nw = small <= kSmallSpreadWaves ? 1 : kWriteWaves;
     paged_write_small_kernel<D, MODE, BF, PROBE>
         <<<((int)small + nw - 1) / nw, nw * kWave, 0, l.stream>>>(a);

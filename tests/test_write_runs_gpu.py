@@ -98,3 +98,17 @@ def test_write_runs(tokens, hkv, head_dim, block_size, mode, breaks):
         g = g.cpu().numpy()
         bad = np.argwhere(g.view(np.uint8).reshape(-1) != w.view(np.uint8).reshape(-1))
         assert bad.size == 0, f"{name}: {len(bad)} bytes differ, first at byte {bad[0][0]}"
+
+
+# (tokens, kv heads) on both sides of where the few-rows form ends: 2048 waves (fp16, head_dim
+# 256), 3072 (fp16; INT8 at 256) and 4096 (INT8), two per window and head; 704, one-wave work-groups
+@pytest.mark.parametrize("breaks", [False, True])
+@pytest.mark.parametrize("mode", ["int8", "fp16"])
+@pytest.mark.parametrize("head_dim,tokens,hkv", [(256, 2048, 8), (256, 2049, 8), (256, 3072, 8),
+                                                 (256, 3073, 8), (128, 12288, 2), (128, 12289, 2),
+                                                 (128, 16384, 2), (128, 16385, 2), (128, 2816, 2),
+                                                 (128, 2817, 2)])
+def test_write_runs_at_the_forms_edges(head_dim, tokens, hkv, mode, breaks):
+    if tokens > 1000 and head_dim == 256:
+        tokens, hkv = 4 * tokens - 4, hkv // 4       # (as test_write_runs maps them back)
+    test_write_runs(tokens, hkv, head_dim, 16, mode, breaks)
