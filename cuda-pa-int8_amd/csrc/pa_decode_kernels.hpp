@@ -1526,6 +1526,8 @@ struct SchedArgs {
   int pmin, pmax;     // partition bounds (multiples of kIterTokens)
   int pmin_uniform;   // lower bound when all lengths are equal (one item per work-group)
   float fill_scale;   // 1024 * kv heads * head chunks / CUs (see the ragged floor below)
+  int equal_items;    // items of a unit that fill one round of the CUs; 0: equal_partition
+                      // does not apply (more units than CUs, a forced partition)
 };
 
 constexpr int kShortBuckets = 4;   // (their counts pack into one 64-bit word)
@@ -1653,7 +1655,6 @@ __device__ __forceinline__ uint32_t wave_scan_dpp(uint32_t v) {
 __device__ __forceinline__ uint32_t equal_partition(const DecodeShape& sh, const SchedArgs& sa,
                                                     int cus, uint32_t b) {
   const uint32_t units = (uint32_t)(sh.num_seqs * sh.num_kv_heads * sh.nchunk);
-  if (units > (uint32_t)cus || sa.pmin >= sa.pmax) return 0;   // (forced partitions stay)
   const uint32_t lo = (uint32_t)sa.pmin_uniform, hi = (uint32_t)sa.pmax;
   // (reciprocals instead of integer divisions, each a long sequence at the start of
   // every launch; the half and the last step make up for their rounding)
@@ -1711,7 +1712,8 @@ __device__ __forceinline__ Schedule build_schedule_small(const int* __restrict__
     f = (f + kIterTokens - 1) / kIterTokens * kIterTokens;
     const uint64_t lo = (sc.uniform || f < (uint64_t)sa.pmin_uniform) ? (uint64_t)sa.pmin_uniform : f;
     part = part < lo ? lo : (part > (uint64_t)sa.pmax ? (uint64_t)sa.pmax : part);
-    if (sc.uniform) {
+    // (where the units divide the CUs, the partition above is that one already)
+    if (sc.uniform && sa.equal_items != 0 && part * (uint32_t)sa.equal_items < b) {
       const uint32_t eq =
           equal_partition(sh, sa, (int)((gridDim.x + kGroupsPerCU - 1) / kGroupsPerCU), b);
       if (eq != 0) part = eq;
@@ -2398,9 +2400,11 @@ hipError_t launch_decode_tiles(const DecodeLaunch& l) {
   if (l.sched) {
     constexpr int kGroupsPerCU = kWavesPerCU / NW;
     const int cus = (l.groups + kGroupsPerCU - 1) / kGroupsPerCU;
+    const long long units = (long long)l.shape.num_seqs * l.shape.num_kv_heads * l.shape.nchunk;
     const SchedArgs sa{l.queue, l.rows_max, l.pmin, l.pmax, l.pmin_uniform,
                        1024.f * (float)(l.shape.num_kv_heads * l.shape.nchunk) /
-                           (float)(cus > 0 ? cus : 1)};
+                           (float)(cus > 0 ? cus : 1),
+                       units > 0 && units <= cus && l.pmin < l.pmax ? cus / (int)units : 0};
     const auto* q = static_cast<const half_t*>(l.q);
     const auto* kc = static_cast<const uint8_t*>(l.k_cache);
     const auto* vc = static_cast<const uint8_t*>(l.v_cache);
