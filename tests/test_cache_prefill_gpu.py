@@ -103,11 +103,10 @@ def test_every_tensor_scale():
     import pa_int8
 
     for dtype in (torch.float16, torch.bfloat16):
-        mags = torch.arange(0, 1 << 15, 7, dtype=torch.int16).view(dtype).to(DEV)
+        mags = torch.arange(0, 1 << 15, dtype=torch.int32).to(torch.int16).view(dtype).to(DEV)
         c = pa_int8.PagedKVCache(1, 1, 8, 16, variant="int8_per_tensor", device=DEV)
         got = []
-        for m in mags:
-            x = m.expand(1, 1, 8).contiguous()
+        for x in mags.view(-1, 1, 1, 1).expand(-1, 1, 1, 8).contiguous():
             c.prefill(0, x, x)
             got.append(c._k_tensor_scale[0])
         got = torch.cat(got)

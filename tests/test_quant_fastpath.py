@@ -73,6 +73,35 @@ def test_scale_by_multiplication_equals_division():
     assert np.array_equal(by_mul.view(np.uint16), by_div.view(np.uint16))
 
 
+def test_tensor_scale_by_multiplication_equals_division():
+    """The per-tensor scale, t(a / 127) for t = fp16 or bf16, by the scales kernel's product
+    (fp16 by the conversion, bf16 by rounding its bits to nearest even) equals torch's for
+    all 32768 magnitudes of both types, infinity and NaN included."""
+    import torch
+
+    bits = np.arange(1 << 15, dtype=np.uint16)
+    inv = np.float32(1) / np.float32(127)
+
+    def clamped(s):
+        return np.where(s < np.float32(1e-8), np.float32(1e-8), s)      # NaN stays
+
+    h = bits.view(np.float16).astype(np.float32)
+    with np.errstate(invalid="ignore"):
+        fp16 = clamped((h * inv).astype(np.float16).astype(np.float32))
+    f = (bits.astype(np.uint32) << 16).view(np.float32)
+    with np.errstate(invalid="ignore", under="ignore"):
+        q = f * inv
+    b = q.view(np.uint32).astype(np.uint64)
+    r = np.where(np.isnan(q), (b >> 16) | 0x40, (b + 0x7FFF + ((b >> 16) & 1)) >> 16)
+    bf16 = clamped((r.astype(np.uint32) << 16).view(np.float32))
+    for got, dtype in ((fp16, torch.float16), (bf16, torch.bfloat16)):
+        mags = torch.from_numpy(bits.view(np.int16)).view(dtype)
+        want = (mags / 127.0).to(torch.float32).clamp_min(1e-8).numpy()
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        ok = ~np.isnan(want)
+        assert np.array_equal(got[ok], want[ok]), dtype
+
+
 def test_group_max_equals_per_element_test():
     """The kernel tests the largest |y - rint(y)| of a group once; on finite
     values that is the per-element test taken over the group."""
