@@ -173,3 +173,37 @@ def plan(seqs, heads, kv_heads, d, bs, blocks, int8):
     assert lib.pa_decode_plan_detail(3 if int8 else 1, seqs, heads, d, kv_heads, bs, blocks, 0, 0,
                                      info, 7) == 0
     return list(info)
+
+
+@pytest.mark.parametrize("int8", [False, True])
+@pytest.mark.parametrize("equal", [False, True])
+def test_partition_under_a_lowered_row_capacity(equal, int8):
+    """The no-alloc entry, whose static scratch holds fewer rows than the schedule asks for
+    (eight head chunks of 128 query heads on one kv head): the same items, to the bit."""
+    import pa_int8
+
+    lib = pa_int8.capi()
+    seqs, heads, d, bs = 17, 128, 256, 16
+    g = torch.Generator().manual_seed(5)
+    lens = [5001] * seqs if equal else torch.randint(900, 9000, (seqs,), generator=g).tolist()
+    kind = 3 if int8 else 1
+    info = plan(seqs, heads, 1, d, bs, -(-max(lens) // bs), int8)
+    assert heads // info[3] == 8
+    assert lib.pa_decode_workspace_bytes(kind, seqs, heads, d, 1, bs, -(-max(lens) // bs), 0,
+                                         0) > 64 << 20
+    x = case(lens, heads, 1, d, bs, int8)
+    q, kc, vc, sc, bt, ctx = x
+    if equal:
+        want = equal_partition(lens[0], seqs, 1, 8, int8, d, info[2])
+    else:
+        want = ragged_partition(lens, 1, 8, int8, d, info[2])
+    check(x, lens, bs, int8, want)
+    out = torch.full_like(q, float("nan"))
+    st = lib.pa_paged_decode_attn_noalloc(
+        kind, out.data_ptr(), q.data_ptr(), kc.data_ptr(), vc.data_ptr(),
+        sc[0].data_ptr() if int8 else None, sc[1].data_ptr() if int8 else None, bt.data_ptr(),
+        ctx.data_ptr(), d ** -0.5, bs, seqs, heads, d, 1, kc.shape[0], 8, bt.shape[1], 0, 0,
+        torch.cuda.current_stream().cuda_stream)
+    assert st == 0, lib.pa_status_string(st)
+    same = torch.equal(out, run(x, bs, int8))
+    assert same
