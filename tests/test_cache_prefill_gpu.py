@@ -126,3 +126,34 @@ def test_empty_prompt():
     c = pa_int8.PagedKVCache(1, 2, 64, 64, variant="int8_per_tensor", device=DEV)
     with pytest.raises(RuntimeError):
         c.prefill(0, e, e)
+
+
+@pytest.mark.parametrize("variant", ["fp16", "int8_per_token", "int8_per_tensor"])
+def test_prefill_under_capture(variant):
+    """A captured prefill replayed over new rows in the same buffers, with eager prefills and
+    synchronizations in between: each replay equals the eager result."""
+    import pa_int8
+
+    tokens, hkv, d = 333, 2, 128
+    k, v = (torch.empty(tokens, hkv, d, dtype=torch.float16, device=DEV) for _ in range(2))
+    cap, ref = (pa_int8.PagedKVCache(1, hkv, d, 512, variant=variant, device=DEV) for _ in range(2))
+    k.normal_(), v.normal_()
+    cap.prefill(0, k, v)                      # (warm-up outside the capture)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        cap.prefill(0, k, v)
+    for i in range(4):
+        g = torch.Generator(device=DEV).manual_seed(i)
+        k.normal_(generator=g), v.normal_(generator=g)
+        k.mul_(1.0 + i)
+        for t in cap._tensors() + ref._tensors():
+            t.fill_(5)
+        graph.replay()
+        torch.cuda.synchronize()
+        ref.prefill(0, k, v)
+        for a, b in zip(cap._tensors(), ref._tensors()):
+            assert torch.equal(bits(a), bits(b)), i
+        if variant == "int8_per_tensor":
+            assert torch.equal(cap._k_tensor_scale[0], ref._k_tensor_scale[0])
+            assert torch.equal(cap._v_tensor_scale[0], ref._v_tensor_scale[0])
